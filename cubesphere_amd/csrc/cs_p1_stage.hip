@@ -854,7 +854,7 @@ __device__ __forceinline__ void face_points(const Dev& D, int fam, int s, int i,
 // centroid, the reciprocal scale length) and its value at a point, with the
 // arithmetic of face_points.
 constexpr int kFpTI = 16, kFpTJ = 8;  // columns per workgroup along i and j
-constexpr int kFpLevels = 16;         // levels per workgroup at most
+constexpr int kFpLevels = 8;          // levels per workgroup at most (march_levels)
 constexpr int kBWords = 16;
 __device__ __forceinline__ void b_at(const double* w, const double* p, double* b) {
   double r[3];
@@ -881,7 +881,7 @@ __device__ __forceinline__ void lds_b(const double (*Bs)[kFpTI * kFpTJ], int slo
 //
 // The faces' geometry (about 60 words of angular tables per column) is the
 // same at every level, and one workgroup reads it again at each level; the
-// march is split into chunks of nlev levels, and the chunks of one block of
+// march is split into chunks of nlev levels (march_levels), and the chunks of one block of
 // columns are consecutive workgroups of one XCD, so they run together and
 // read the tables through that XCD's L2 instead of HBM.  A chunk after the
 // first takes the zone below its first z-face from memory.
@@ -1472,7 +1472,11 @@ __device__ __forceinline__ void face_solve(const Dev& D, int fam, int s, int k, 
 // L2; a chunk after the first starts one level early with its faces off, so
 // that level leaves the bottom state of the chunk's first z-face.
 constexpr int kFluxTI = 16, kFluxTJ = 8;  // columns per workgroup along i and j
-constexpr int kFluxLevels = 16;           // levels per workgroup at most
+// levels per workgroup at most (march_levels): 4, and 16 where the tables
+// (about 35 words a column) no longer fit the 256 MB Infinity Cache and a
+// chunk's levels must share one fetch of them
+constexpr int kFluxLevels = 4, kFluxLevelsBig = 16;
+constexpr int64_t kInfinityCache = 256 << 20;
 constexpr int kSlopeWords = 40;           // 4 x 9 modes, the centroid, the reciprocal scale length
 __device__ __forceinline__ void lds_state(const double (*Zs)[kFluxTI * kFluxTJ], int slot, const double* p,
                                           double* w) {
@@ -2362,6 +2366,22 @@ int create(const cs_config* cfg, Stage** out, size_t* bytes) {
   return CS_OK;
 }
 
+// Levels per workgroup of a column march over `levels` levels, `blocks`
+// blocks of columns in all sectors: as many as leave about kMarchBlocks
+// workgroups, between 1 and `most`.  A workgroup's levels run one after the
+// other, so on a small shell a long march leaves most of the chip idle and
+// its time is that of one chain; above some 4000 workgroups (256 CUs, four
+// to a CU, four waves of them) more chunks only repeat lead-in levels.
+// k_face_pts / k_flux, us per launch, all levels up to 16 in one chunk ->
+// this rule: 24^2 x 8 183 / 252 -> 36 / 40, 45^2 x 17 184 / 291 -> 82 / 114,
+// 64^2 x 24 274 / 457 -> 198 / 250, 96^2 x 32 479 / 771 -> 439 / 618,
+// 160^2 x 48 1599 / 2325 -> 1578 / 2261; 512^2 x 128 keeps 36.1 / 54.0 ms
+// (k_flux with chunks of 4: 55.6 ms).
+constexpr int64_t kMarchBlocks = 4096;
+static int march_levels(int levels, int64_t blocks, int most) {
+  return (int)std::max<int64_t>(1, std::min<int64_t>(most, blocks * levels / kMarchBlocks));
+}
+
 static Buf6 b6(const Buf& b) { return Buf6{b.U, b.ent, b.Bx, b.By, b.Bz}; }
 
 int front(Stage* S, const Buf& in_, double* const* F, double* const* Sp, double* const* E, int* err,
@@ -2398,7 +2418,8 @@ int front(Stage* S, const Buf& in_, double* const* F, double* const* Sp, double*
   k_clear_ent<<<dim3(nb(nwr, 256), 6), 256, 0, st>>>(D, S->wr, in, err);
   mark_end(S, st, CS_P1K_REPLAY);
   const int64_t nfpi = (D.N + 7 + kFpTI - 2) / (kFpTI - 1), nfpj = (D.N + 7 + kFpTJ - 2) / (kFpTJ - 1);
-  const int fpl = D.NR + 8, fpch = (fpl + kFpLevels - 1) / kFpLevels, fpnl = (fpl + fpch - 1) / fpch;
+  const int fpl = D.NR + 8, fpm = march_levels(fpl, 6 * nfpi * nfpj, kFpLevels);
+  const int fpch = (fpl + fpm - 1) / fpm, fpnl = (fpl + fpch - 1) / fpch;
   mark_begin(S, st);
   k_face_pts<<<dim3((unsigned)(nfpi * nfpj * fpch), 6), kFpTI * kFpTJ, 0, st>>>(D, in, fpch, fpnl);
   mark_end(S, st, CS_P1K_FACE_POINTS);
@@ -2406,7 +2427,10 @@ int front(Stage* S, const Buf& in_, double* const* F, double* const* Sp, double*
   k_clsq<<<dim3(nb(nall, 64), 6), 64, 0, st>>>(D, S->all, in);
   mark_end(S, st, CS_P1K_CLSQ);
   const int64_t nfi = (D.N + 3 + kFluxTI - 2) / (kFluxTI - 1), nfj = (D.N + 3 + kFluxTJ - 2) / (kFluxTJ - 1);
-  const int fll = D.NR + 4, flch = (fll + kFluxLevels - 1) / kFluxLevels, flnl = (fll + flch - 1) / flch;
+  const int64_t tables = 6 * (int64_t)D.nf * D.nf * 35 * (int64_t)sizeof(double);
+  const int fll = D.NR + 4,
+            flm = march_levels(fll, 6 * nfi * nfj, tables > kInfinityCache ? kFluxLevelsBig : kFluxLevels);
+  const int flch = (fll + flm - 1) / flm, flnl = (fll + flch - 1) / flch;
   mark_begin(S, st);
   k_flux<<<dim3((unsigned)(nfi * nfj * flch), 6), kFluxTI * kFluxTJ, 0, st>>>(D, F[0], F[1], F[2], Sp[0], Sp[1],
                                                                               Sp[2], flch, flnl);

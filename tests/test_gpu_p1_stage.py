@@ -13,8 +13,8 @@ Cases named for the benchmark configurations they shrink:
       layers by PAD_BOUNDARY_R, outflow at both ends, and, in a second case,
       by ADD_BOUNDARY with the problem's own state);
   plus the reference's own combination (HLL, Heun RK2) on a shell, a
-  6x8^2x20 shell tall enough that the face kernels split every column's
-  march into two chunks of levels, and a blast with log-normal noise so the
+  6x8^2x20 shell whose columns the face kernels march in one-level chunks,
+  and a blast with log-normal noise so the
   positivity limiter removes slopes and its loop-order replay runs on the
   device.
 
@@ -166,6 +166,30 @@ def test_p1_stage_matches_oracle(name):
     print(f"case {name}: rel L1 {w:.2e}, div B {np.abs(d0).max():.2e}, its change over two steps {change:.2e}")
     # constrained transport: each zone's discrete divergence changes only by rounding
     assert change < 1e-12
+
+
+def test_p1_stage_march_chunks():
+    """A shell with enough blocks of columns that the face kernels march two
+    levels per workgroup, the last chunk of one level (48^2 x 41: 192 blocks of
+    15 x 7 columns, 45 levels of k_flux and 49 of k_face_pts): one step
+    against the oracle.  The smaller shells of this file march one level each."""
+    cfg = cs.make_config(48, 41, 4, cs.RECON_P1ADP, cs.RS_HLLD, cs.EMF_LLF, cs.FP64, 2, cs.RBC_PAD, cs.RMESH_UNIFORM,
+                         1.0, 1.5)
+    st0 = _state(cfg, 3, 0.0)
+    ref = st0.copy()
+    print("march chunks: oracle step", flush=True)
+    dt1 = orc.p1s_step_oracle(orc.Grid(cfg), cfg, orc.p1s_patches(cfg), ref, 1e-3)
+    print("march chunks: device step", flush=True)
+    h = cs.CubeSphere(cfg)
+    try:
+        h.upload(st0)
+        h.dt = 1e-3
+        h.advance(1)
+        got = h.download()
+        assert abs(h.dt - dt1) <= 1e-9 * dt1
+    finally:
+        h.close()
+    _compare(cfg, got, ref, 1e-9)
 
 
 def test_p1_stage_graph_equals_eager():
