@@ -53,11 +53,11 @@ void set_error(const char* fmt, ...);
 namespace p1s {
 
 constexpr int kSweeps = 12;          // bound on the positivity replay sweeps per stage
-constexpr int kListBlocks = 1024;    // grid of the list kernels (grid-stride)
+constexpr int kListBlocks = 512;     // grid of the replay kernels (grid-stride)
 constexpr int kCflBlocks = 1024;     // grid of the time-step reduction
 // counters: [0] zones whose slopes pass 0 removed, [1] list length,
-// [2] settled, [3 .. 3 + kSweeps) flag changes per sweep
-constexpr int kCtr = 3 + kSweeps;
+// [2 .. 2 + kSweeps) flag changes per sweep
+constexpr int kCtr = 2 + kSweeps;
 
 struct Dev {
   int N, NR, g, nz, nzr, nf, nfr;
@@ -70,7 +70,7 @@ struct Dev {
   int64_t NZB;             // zone blocks of 64 per sector
   double *flat, *work, *ms;  // [s][zone]
   double* Bq;              // [s][fam][5][face]: normal B at the B-field points
-  uint8_t *fa, *prev, *next, *ever, *inlist;  // [s][zone]
+  uint8_t *fl[2], *ever, *inlist;  // [s][zone]; sweep n of the replay reads fl[n % 2], writes fl[(n + 1) % 2]
   uint32_t* list;          // packed s * NZ + zone
   unsigned int* ctr;
   double gamma, rhofloor, prsfloor, smallnum, flatten_coef, prs_flatten_coef, grav;
@@ -265,31 +265,33 @@ __global__ void __launch_bounds__(256) k_prim(Dev D, Box b, Buf6 in) {
   }
 }
 
-// step 2 (faces): face B between two inactive zones cleared; blockIdx.y = fam + 3 s
-__global__ void __launch_bounds__(256) k_face_zero(Dev D, Buf6 in) {
-  const int fam = blockIdx.y % 3, s = blockIdx.y / 3;
-  const int64_t t = tid();
-  if (t >= D.NFC) return;
-  const int n = D.nf;
-  const int i = (int)(t % n) - D.g, j = (int)((t / n) % n) - D.g, k = (int)(t / ((int64_t)n * n)) - D.g;
-  const int lo = 1 - D.g, hi = D.N + D.g, hr = D.NR + D.g;
-  double* B = in.b(fam) + (int64_t)s * D.NFC;
+// steps 2 and 3 for the face B, which meet on no face: blockIdx.y = fam + 3 s
+// < 18 clears the faces between two inactive zones (only tri-corner columns
+// hold inactive zones, so the work items are the faces of those four blocks:
+// 4 (g + 1)^2 columns instead of all (N + 2 g + 1)^2), blockIdx.y - 18 = s
+// synchronises the face B at the sector's tri-corners.  One launch instead
+// of two over all faces: 256^2 surface 35.2 -> 6.7 us, 160^2 x 48 shell
+// 73.8 -> 8.5 us (what is left is launch latency).
+__device__ __forceinline__ void face_zero(const Dev& D, const Buf6& in, int fam, int s, int64_t t) {
+  const int w = 2 * (D.g + 1), g = D.g;
+  if (t >= (int64_t)w * w * D.nfr) return;
+  const int a = (int)(t % w), b = (int)((t / w) % w), k = (int)(t / ((int64_t)w * w)) - g;
+  const int i = a <= g ? a - g : D.N + a - g - 1, j = b <= g ? b - g : D.N + b - g - 1;
+  const int lo = 1 - g, hi = D.N + g, hr = D.NR + g;
+  double* B = in.b(fam) + (int64_t)s * D.NFC + D.fci(i, j, k);
   if (fam == 0) {
     if (j < lo || k < lo || k > hr) return;
-    if (!D.active(max(i, lo), j) && !D.active(min(i + 1, hi), j)) B[t] = 0.0;
+    if (!D.active(max(i, lo), j) && !D.active(min(i + 1, hi), j)) *B = 0.0;
   } else if (fam == 1) {
     if (i < lo || k < lo || k > hr) return;
-    if (!D.active(i, max(j, lo)) && !D.active(i, min(j + 1, hi))) B[t] = 0.0;
+    if (!D.active(i, max(j, lo)) && !D.active(i, min(j + 1, hi))) *B = 0.0;
   } else {
     if (i < lo || j < lo) return;
-    if (!D.active(i, j)) B[t] = 0.0;
+    if (!D.active(i, j)) *B = 0.0;
   }
 }
-
-// step 3: face B synchronised at the four tri-corners of every sector
-__global__ void __launch_bounds__(256) k_tricorner(Dev D, Buf6 in) {
-  const int64_t t = tid();
-  const int g = D.g, nzr = D.nzr, s = blockIdx.y;
+__device__ __forceinline__ void tricorner(const Dev& D, const Buf6& in, int s, int64_t t) {
+  const int g = D.g, nzr = D.nzr;
   if (t >= 4 * (int64_t)g * nzr) return;
   const int corner = (int)(t / ((int64_t)g * nzr)), ii = (int)((t / nzr) % g), k = (int)(t % nzr) + 1 - g;
   const bool left = corner == 0 || corner == 3, down = corner < 2;
@@ -307,6 +309,10 @@ __global__ void __launch_bounds__(256) k_tricorner(Dev D, Buf6 in) {
     by = h;
     bx = h;
   }
+}
+__global__ void __launch_bounds__(256) k_face_sync(Dev D, Buf6 in) {
+  if (blockIdx.y < 18) face_zero(D, in, blockIdx.y % 3, blockIdx.y / 3, tid());
+  else tricorner(D, in, blockIdx.y - 18, tid());
 }
 
 // ---------------------------------------------------------------------------
@@ -365,6 +371,8 @@ __global__ void __launch_bounds__(256) k_flat_a(Dev D, Box b) {
 __global__ void __launch_bounds__(256) k_flat_b(Dev D, Box b) {
   int i, j, k;
   const LBlock wg = lblock();
+  // the replay's counters start at zero (read and counted from k_pos on)
+  if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x < kCtr) D.ctr[threadIdx.x] = 0;
   if (!b.decode(ltid(wg), i, j, k)) return;
   const int s = wg.y;
   const int64_t z = D.zi(i, j, k), so = (int64_t)s * D.NZ;
@@ -538,26 +546,12 @@ __global__ void __launch_bounds__(128) k_weno(Dev D, Box b) {
     for (int m = 0; m < 3; ++m) D.v(m + 1, s, f, z) = (num[m] + w8 * X8[m]) * os * omf;
   }
 }
-// the zones of the replay list (grid-stride)
-__global__ void __launch_bounds__(128) k_weno_list(Dev D) {
-  if (D.ctr[0] == 0 || D.ctr[2]) return;
-  const int64_t n = D.ctr[1];
-  for (int64_t t = tid(); t < 3 * n; t += (int64_t)gridDim.x * blockDim.x) {
-    const uint32_t p = D.list[t % n];
-    const int s = (int)(p / D.NZ);
-    const int64_t z = p - (int64_t)s * D.NZ;
-    int i, j, k;
-    D.zone_of(z, i, j, k);
-    weno3(D, s, i, j, k, z, 3 * (int)(t / n));
-  }
-}
-
 // ---------------------------------------------------------------------------
 // step 7.b: ENFORCE_PRESSURE_POSITIVITY_PRIM (440...f:6-830).  pass < 0: the
 // first pass over the range with the incoming entropy means; flags of every
 // zone set, zones whose slopes were removed counted.  pass >= 0: replay sweep
-// `pass` on the list, taking the entropy means of earlier zones whose prev
-// flag is set as zero (440...f:553-560), flag changes counted.
+// `pass` on the list, taking the entropy means of earlier zones whose
+// previous flag is set as zero (440...f:553-560), flag changes counted.
 __device__ __forceinline__ void columns9(const Dev& D, int i, int j, int64_t* c9) {
   c9[0] = D.zi(i, j, 0);
   const int dirs[8] = {0, 1, 2, 3, 8, 9, 10, 11};
@@ -582,7 +576,7 @@ __device__ __forceinline__ void positivity(const Dev& D, int s, int i, int j, in
       const int64_t zz = c9[q] + ks * (k + dk);
       const double r = D.v(0, s, 0, zz), p = D.v(0, s, 4, zz);
       double e = D.v(0, s, 8, zz);
-      if (pass >= 0 && zz < z && D.prev[so + zz]) e = 0.0;
+      if (pass >= 0 && zz < z && D.fl[pass & 1][so + zz]) e = 0.0;
       rmin = fmin(rmin, r);
       rmax = fmax(rmax, r);
       pmin = fmin(pmin, p);
@@ -709,15 +703,15 @@ __device__ __forceinline__ void positivity(const Dev& D, int s, int i, int j, in
   }
   const uint8_t flag = removed ? 1 : 0;
   if (pass < 0) {
-    D.fa[so + z] = flag;
-    D.prev[so + z] = flag;
-    D.next[so + z] = flag;
+    D.fl[0][so + z] = flag;
+    D.fl[1][so + z] = flag;
     D.ever[so + z] = flag;
     D.inlist[so + z] = 0;
     if (removed) atomicAdd(&D.ctr[0], 1u);
   } else {
-    D.next[so + z] = flag;
-    if (flag != D.prev[so + z]) atomicAdd(&D.ctr[3 + pass], 1u);
+    D.fl[(pass + 1) & 1][so + z] = flag;
+    if (flag) D.ever[so + z] = 1;
+    if (flag != D.fl[pass & 1][so + z]) atomicAdd(&D.ctr[2 + pass], 1u);
   }
 }
 __global__ void __launch_bounds__(256) k_pos(Dev D, Box b) {
@@ -726,69 +720,83 @@ __global__ void __launch_bounds__(256) k_pos(Dev D, Box b) {
   if (!b.decode(ltid(wg), i, j, k)) return;
   positivity(D, wg.y, i, j, k, D.zi(i, j, k), -1);
 }
-__global__ void __launch_bounds__(256) k_pos_list(Dev D, int sweep) {
-  if (D.ctr[0] == 0 || D.ctr[2]) return;
-  const int64_t n = D.ctr[1];
-  for (int64_t t = tid(); t < n; t += (int64_t)gridDim.x * blockDim.x) {
-    const uint32_t p = D.list[t];
-    const int s = (int)(p / D.NZ);
-    const int64_t z = p - (int64_t)s * D.NZ;
-    int i, j, k;
-    D.zone_of(z, i, j, k);
-    positivity(D, s, i, j, k, z, sweep);
-  }
-}
-__global__ void k_ctr_reset(Dev D) {
-  if (threadIdx.x < kCtr) D.ctr[threadIdx.x] = 0;
+// The replay, two launches a sweep.  A sweep after one that changed no flag
+// has nothing to do, and its own change count, zero since k_flat_b, passes
+// that on; without removed zones (ctr[0] == 0) no sweep does anything.
+__device__ __forceinline__ bool replay_done(const Dev& D, int sweep) {
+  return D.ctr[0] == 0 || (sweep > 0 && D.ctr[2 + sweep - 1] == 0);
 }
 // the zones of the range with a zone ever flagged earlier in the loop order
 // among their 27 join the list (each once: the list only grows, so a zone
-// that depends on a flag is recomputed in every later sweep)
-__global__ void __launch_bounds__(256) k_cands(Dev D, Box b) {
-  if (D.ctr[0] == 0 || D.ctr[2]) return;
-  int i, j, k;
-  if (!b.decode(tid(), i, j, k)) return;
-  const int s = blockIdx.y;
-  const int64_t z = D.zi(i, j, k), so = (int64_t)s * D.NZ, ks = (int64_t)D.nz * D.nz;
-  if (D.inlist[so + z]) return;
-  int64_t c9[9];
-  columns9(D, i, j, c9);
-  bool cand = false;
-  for (int q = 0; q < 9; ++q)
+// that depends on a flag is recomputed in every later sweep; both flag
+// arrays of a zone that joins still hold its first pass's flag).
+// Grid-stride over the six sectors: an idle sweep costs a small launch
+// whatever the shell's size.
+__global__ void __launch_bounds__(256) k_cands(Dev D, Box b, int sweep) {
+  if (replay_done(D, sweep)) return;
+  const int64_t n = b.count(), ks = (int64_t)D.nz * D.nz;
+  for (int64_t t = tid(); t < 6 * n; t += (int64_t)gridDim.x * blockDim.x) {
+    int i, j, k;
+    const int s = (int)(t / n);
+    b.decode(t - s * n, i, j, k);
+    const int64_t z = D.zi(i, j, k), so = (int64_t)s * D.NZ;
+    if (D.inlist[so + z]) continue;
+    int64_t c9[9];
+    columns9(D, i, j, c9);
+    bool cand = false;
+    for (int q = 0; q < 9; ++q)
 #pragma unroll
-    for (int dk = -1; dk <= 1; ++dk) {
-      const int64_t zz = c9[q] + ks * (k + dk);
-      cand = cand || (zz < z && D.ever[so + zz]);
+      for (int dk = -1; dk <= 1; ++dk) {
+        const int64_t zz = c9[q] + ks * (k + dk);
+        cand = cand || (zz < z && D.ever[so + zz]);
+      }
+    if (cand) {
+      D.inlist[so + z] = 1;
+      D.list[atomicAdd(&D.ctr[1], 1u)] = (uint32_t)(so + z);
     }
-  if (cand) {
-    D.inlist[so + z] = 1;
-    D.list[atomicAdd(&D.ctr[1], 1u)] = (uint32_t)(so + z);
   }
 }
-// end of a sweep: the new flags become the previous ones; no change: settled
-__global__ void __launch_bounds__(256) k_commit(Dev D, int sweep) {
-  if (D.ctr[0] == 0) return;
+// the list's zones in groups of 64: three waves redo their WENO (three fields
+// each), then the first wave their positivity.  The replay was 48 launches a
+// stage (candidates, WENO, positivity and the flags' commit in each of the 12
+// sweeps) and is 24 small ones.  Idle, it costs their latency: 24^2 x 8
+// 81 -> 43 us, 160^2 x 48 180 -> 46 us; the 256^2 blast surface, where it
+// has zones to redo, 107 -> 78 us.
+constexpr int kReplayZones = 64;
+__global__ void __launch_bounds__(3 * kReplayZones) k_replay(Dev D, int sweep) {
+  if (replay_done(D, sweep)) return;
   const int64_t n = D.ctr[1];
-  for (int64_t t = tid(); t < n; t += (int64_t)gridDim.x * blockDim.x) {
-    const uint32_t p = D.list[t];
-    const uint8_t f = D.next[p];
-    D.prev[p] = f;
-    D.ever[p] = D.ever[p] | f;
+  const int q = threadIdx.x % kReplayZones, grp = threadIdx.x / kReplayZones;
+  for (int64_t t0 = (int64_t)blockIdx.x * kReplayZones; t0 < n; t0 += (int64_t)gridDim.x * kReplayZones) {
+    const bool on = t0 + q < n;
+    int s = 0, i = 0, j = 0, k = 0;
+    int64_t z = 0;
+    if (on) {
+      const uint32_t p = D.list[t0 + q];
+      s = (int)(p / D.NZ);
+      z = p - (int64_t)s * D.NZ;
+      D.zone_of(z, i, j, k);
+      weno3(D, s, i, j, k, z, 3 * grp);
+    }
+    __syncthreads();  // the zone's slopes are written before its positivity reads them
+    if (on && grp == 0) positivity(D, s, i, j, k, z, sweep);
   }
-  if (tid() == 0 && D.ctr[3 + sweep] == 0) D.ctr[2] = 1;
 }
 // after the sweeps: the entropy means of the zones that lost their slopes
 // are zero (440...f:553-560); a replay that has not settled is an error
 __global__ void __launch_bounds__(256) k_clear_ent(Dev D, Box b, Buf6 in, int* err) {
   if (D.ctr[0] == 0) return;
-  if (tid() == 0 && blockIdx.y == 0 && !D.ctr[2]) atomicOr(err, 1);
-  int i, j, k;
-  if (!b.decode(tid(), i, j, k)) return;
-  const int s = blockIdx.y;
-  const int64_t z = D.zi(i, j, k);
-  if (D.prev[(int64_t)s * D.NZ + z]) {
-    in.e(D, s, z) = 0.0;
-    D.v(0, s, 8, z) = 0.0;
+  if (tid() == 0 && D.ctr[2 + kSweeps - 1] != 0) atomicOr(err, 1);
+  const int64_t n = b.count();
+  for (int64_t t = tid(); t < 6 * n; t += (int64_t)gridDim.x * blockDim.x) {
+    int i, j, k;
+    const int s = (int)(t / n);
+    b.decode(t - s * n, i, j, k);
+    const int64_t z = D.zi(i, j, k);
+    if (D.fl[kSweeps & 1][(int64_t)s * D.NZ + z]) {
+      in.e(D, s, z) = 0.0;
+      D.v(0, s, 8, z) = 0.0;
+    }
   }
 }
 
@@ -2340,8 +2348,8 @@ int create(const cs_config* cfg, Stage** out, size_t* bytes) {
   const int64_t Z6 = 6 * D.NZ;
   if ((rc = dalloc(S, D.V, 6 * 36 * 64 * D.NZB, bytes)) || (rc = dalloc(S, D.flat, Z6, bytes)) ||
       (rc = dalloc(S, D.work, Z6, bytes)) || (rc = dalloc(S, D.ms, Z6, bytes)) ||
-      (rc = dalloc(S, D.Bq, 6 * 3 * 5 * D.NFC, bytes)) || (rc = dalloc(S, D.fa, Z6, bytes)) ||
-      (rc = dalloc(S, D.prev, Z6, bytes)) || (rc = dalloc(S, D.next, Z6, bytes)) ||
+      (rc = dalloc(S, D.Bq, 6 * 3 * 5 * D.NFC, bytes)) || (rc = dalloc(S, D.fl[0], Z6, bytes)) ||
+      (rc = dalloc(S, D.fl[1], Z6, bytes)) ||
       (rc = dalloc(S, D.ever, Z6, bytes)) || (rc = dalloc(S, D.inlist, Z6, bytes)) ||
       (rc = dalloc(S, D.list, Z6, bytes)) || (rc = dalloc(S, D.ctr, 64, bytes)))
     return fail(rc);
@@ -2393,14 +2401,12 @@ int front(Stage* S, const Buf& in_, double* const* F, double* const* Sp, double*
   k_prim<<<dim3(nb(nall, 256), 6), 256, 0, st>>>(D, S->all, in);
   mark_end(S, st, CS_P1K_PRIM);
   mark_begin(S, st);
-  k_face_zero<<<dim3(nb(D.NFC, 256), 18), 256, 0, st>>>(D, in);
-  k_tricorner<<<dim3(nb(4 * (int64_t)D.g * D.nzr, 256), 6), 256, 0, st>>>(D, in);
+  k_face_sync<<<dim3(nb(4 * (int64_t)(D.g + 1) * (D.g + 1) * D.nfr, 256), 24), 256, 0, st>>>(D, in);
   mark_end(S, st, CS_P1K_FACE_SYNC);
   mark_begin(S, st);
   k_flat_a<<<dim3(tile_blocks<32, 8>(S->all), 6), 256, 0, st>>>(D, S->all);
   k_flat_b<<<dim3(nb(nall, 256), 6), 256, 0, st>>>(D, S->all);
   k_flat_c<<<dim3(nb(nall, 256), 6), 256, 0, st>>>(D, S->all);
-  k_ctr_reset<<<1, 64, 0, st>>>(D);
   mark_end(S, st, CS_P1K_FLATTEN);
   mark_begin(S, st);
   k_weno<<<dim3(nb(nwr, 128), 6), 128, 0, st>>>(D, S->wr);
@@ -2410,12 +2416,10 @@ int front(Stage* S, const Buf& in_, double* const* F, double* const* Sp, double*
   mark_end(S, st, CS_P1K_POSITIVITY);
   mark_begin(S, st);
   for (int sw = 0; sw < kSweeps; ++sw) {
-    k_cands<<<dim3(nb(nwr, 256), 6), 256, 0, st>>>(D, S->wr);
-    k_weno_list<<<kListBlocks, 128, 0, st>>>(D);
-    k_pos_list<<<kListBlocks, 256, 0, st>>>(D, sw);
-    k_commit<<<kListBlocks, 256, 0, st>>>(D, sw);
+    k_cands<<<kListBlocks, 256, 0, st>>>(D, S->wr, sw);
+    k_replay<<<kListBlocks, 3 * kReplayZones, 0, st>>>(D, sw);
   }
-  k_clear_ent<<<dim3(nb(nwr, 256), 6), 256, 0, st>>>(D, S->wr, in, err);
+  k_clear_ent<<<kListBlocks, 256, 0, st>>>(D, S->wr, in, err);
   mark_end(S, st, CS_P1K_REPLAY);
   const int64_t nfpi = (D.N + 7 + kFpTI - 2) / (kFpTI - 1), nfpj = (D.N + 7 + kFpTJ - 2) / (kFpTJ - 1);
   const int fpl = D.NR + 8, fpm = march_levels(fpl, 6 * nfpi * nfpj, kFpLevels);
