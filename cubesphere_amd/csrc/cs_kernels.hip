@@ -21,6 +21,7 @@
 #include "cs_p1_stage.h"
 #include "cs_internal.h"
 #include "cs_dump.h"
+#include "cs_transfer.h"
 #include "cs_physics.h"
 
 using namespace csp;
@@ -1512,6 +1513,7 @@ struct cs_handle {
   int vghost = -1;
   struct Prof* prof = nullptr;  // per-launch event pairs while cs_profile_steps runs
   p1s::Stage* p1 = nullptr;     // the P1 stage's buffers (recon CS_RECON_P1ADP)
+  cs::Staging staging;          // pinned slots of the state's transfers
   int bs[CS_K_COUNT];           // workgroup size per kernel id (cs_autotune)
 };
 
@@ -1904,6 +1906,7 @@ void free_all(cs_handle* h) {
   hipFree(h->dt); hipFree(h->part); hipFree(h->flags);
   p1s::destroy(h->p1);
   h->p1 = nullptr;
+  h->staging.release();
   if (h->stream) hipStreamDestroy(h->stream);
 }
 
@@ -2076,11 +2079,11 @@ extern "C" int cs_upload_state(cs_handle* h, const double* U, const double* ent,
   size_t cb = sizeof(double) * d.cpp * 6, fb = sizeof(double) * d.fpp * 6;
   h->cur = 0;
   h->vbuf = h->vghost = -1;
-  CS_HIP(hipMemcpyAsync(h->buf[0][0], U, cb * 8, hipMemcpyHostToDevice, h->stream));
-  CS_HIP(hipMemcpyAsync(h->buf[0][1], ent, cb, hipMemcpyHostToDevice, h->stream));
-  CS_HIP(hipMemcpyAsync(h->buf[0][2], Bxf, fb, hipMemcpyHostToDevice, h->stream));
-  CS_HIP(hipMemcpyAsync(h->buf[0][3], Byf, fb, hipMemcpyHostToDevice, h->stream));
-  CS_HIP(hipMemcpyAsync(h->buf[0][4], Bzf, fb, hipMemcpyHostToDevice, h->stream));
+  const double* src[5] = {U, ent, Bxf, Byf, Bzf};
+  Segment seg[5];
+  for (int q = 0; q < 5; ++q)
+    seg[q] = Segment{(char*)h->buf[0][q], (char*)const_cast<double*>(src[q]), q == 0 ? cb * 8 : (q == 1 ? cb : fb)};
+  CS_HIP(transfer(h->staging, h->stream, seg, 5, false));
   return finish_upload(h);
 }
 
@@ -2089,13 +2092,13 @@ extern "C" int cs_download_state(cs_handle* h, double* U, double* ent, double* B
   CHECK_H(h);
   const CsDims& d = h->d;
   size_t cb = sizeof(double) * d.cpp * 6, fb = sizeof(double) * d.fpp * 6;
-  int b = h->cur;
-  if (U) CS_HIP(hipMemcpyAsync(U, h->buf[b][0], cb * 8, hipMemcpyDeviceToHost, h->stream));
-  if (ent) CS_HIP(hipMemcpyAsync(ent, h->buf[b][1], cb, hipMemcpyDeviceToHost, h->stream));
-  if (Bxf) CS_HIP(hipMemcpyAsync(Bxf, h->buf[b][2], fb, hipMemcpyDeviceToHost, h->stream));
-  if (Byf) CS_HIP(hipMemcpyAsync(Byf, h->buf[b][3], fb, hipMemcpyDeviceToHost, h->stream));
-  if (Bzf) CS_HIP(hipMemcpyAsync(Bzf, h->buf[b][4], fb, hipMemcpyDeviceToHost, h->stream));
-  CS_HIP(hipStreamSynchronize(h->stream));
+  double* dst[5] = {U, ent, Bxf, Byf, Bzf};
+  Segment seg[5];
+  int n = 0;
+  for (int q = 0; q < 5; ++q)
+    if (dst[q])
+      seg[n++] = Segment{(char*)h->buf[h->cur][q], (char*)dst[q], q == 0 ? cb * 8 : (q == 1 ? cb : fb)};
+  CS_HIP(transfer(h->staging, h->stream, seg, n, true));
   return CS_OK;
 }
 
