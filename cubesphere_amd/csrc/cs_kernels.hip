@@ -1513,7 +1513,6 @@ struct cs_handle {
   int vghost = -1;
   struct Prof* prof = nullptr;  // per-launch event pairs while cs_profile_steps runs
   p1s::Stage* p1 = nullptr;     // the P1 stage's buffers (recon CS_RECON_P1ADP)
-  cs::Staging staging;          // pinned slots of the state's transfers
   int bs[CS_K_COUNT];           // workgroup size per kernel id (cs_autotune)
 };
 
@@ -1906,7 +1905,6 @@ void free_all(cs_handle* h) {
   hipFree(h->dt); hipFree(h->part); hipFree(h->flags);
   p1s::destroy(h->p1);
   h->p1 = nullptr;
-  h->staging.release();
   if (h->stream) hipStreamDestroy(h->stream);
 }
 
@@ -2029,6 +2027,7 @@ extern "C" int cs_create(const cs_config* cfg, cs_handle** out) {
     delete h;
     return CS_E_HIP;
   }
+  staging_pool().enter();
   *out = h;
   return CS_OK;
 }
@@ -2038,6 +2037,7 @@ extern "C" int cs_destroy(cs_handle* h) {
   hipStreamSynchronize(h->stream);
   free_all(h);
   delete h;
+  staging_pool().leave();
   return CS_OK;
 }
 
@@ -2083,7 +2083,7 @@ extern "C" int cs_upload_state(cs_handle* h, const double* U, const double* ent,
   Segment seg[5];
   for (int q = 0; q < 5; ++q)
     seg[q] = Segment{(char*)h->buf[0][q], (char*)const_cast<double*>(src[q]), q == 0 ? cb * 8 : (q == 1 ? cb : fb)};
-  CS_HIP(transfer(h->staging, h->stream, seg, 5, false));
+  CS_HIP(transfer(h->stream, seg, 5, false));
   return finish_upload(h);
 }
 
@@ -2098,7 +2098,7 @@ extern "C" int cs_download_state(cs_handle* h, double* U, double* ent, double* B
   for (int q = 0; q < 5; ++q)
     if (dst[q])
       seg[n++] = Segment{(char*)h->buf[h->cur][q], (char*)dst[q], q == 0 ? cb * 8 : (q == 1 ? cb : fb)};
-  CS_HIP(transfer(h->staging, h->stream, seg, n, true));
+  CS_HIP(transfer(h->stream, seg, n, true));
   return CS_OK;
 }
 

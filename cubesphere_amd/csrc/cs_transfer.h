@@ -1,5 +1,5 @@
 // cs_transfer.h -- copies of a whole state between the caller's (pageable)
-// arrays and the device through the handle's pinned staging slots.
+// arrays and the device through pinned staging slots.
 //
 // The runtime's copy down to pageable memory moves one chunk at a time on the
 // calling thread, and a fresh destination array costs that thread the page
@@ -11,8 +11,7 @@
 // Milliseconds down (into a new array) / up, runtime's copy -> staged: 19 MB
 // 1.4 -> 1.1 / 0.6, 41 MB 3.0 -> 2.0 / 1.4, 109 MB 9.5 -> 3.6 / 3.8 -> 3.1,
 // 232 MB 22.8 -> 6.4 / 7.8 -> 6.2, 864 MB 81 -> 21.8 / 28.6 -> 22.2 (40 GB/s,
-// the link).  The first staged transfer also allocates the slots, 1 to 2 ms,
-// which below the thresholds is more than a few transfers gain.
+// the link).  Below the thresholds the threads cost what they gain.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -20,6 +19,9 @@
 
 #include <algorithm>
 #include <atomic>
+#include <memory>
+#include <mutex>
+#include <new>
 #include <system_error>
 #include <thread>
 
@@ -38,38 +40,77 @@ struct Segment {
   size_t bytes;
 };
 
-// A handle's staging slots (16 to 32 MiB in all), allocated by its first staged
-// transfer for the size of its state, returned with the handle.
+// Pinned slots of one transfer at a time (32 MiB) with their events.
 struct Staging {
   char* pin = nullptr;
-  size_t slot = 0;
+  int device = -1;
   hipEvent_t ev[kSlots] = {};
-  bool ready(size_t total) {
-    if (pin) return true;
-    slot = std::min(kSlotMax, std::max(kSlotMin, total / 16 & ~(size_t)4095));
-    if (hipHostMalloc((void**)&pin, kSlots * slot, hipHostMallocDefault) != hipSuccess) {
-      (void)hipGetLastError();
-      pin = nullptr;
-      return false;
-    }
+  bool make(int dev) {
+    device = dev;
+    bool ok = hipHostMalloc((void**)&pin, kSlots * kSlotMax, hipHostMallocDefault) == hipSuccess;
+    if (!ok) pin = nullptr;
     for (hipEvent_t& e : ev)
-      if (hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) {
-        (void)hipGetLastError();
+      if (ok && hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) {
         e = nullptr;
-        release();
-        return false;
+        ok = false;
       }
-    return true;
+    if (!ok) (void)hipGetLastError();
+    return ok;
   }
-  void release() {
-    for (hipEvent_t& e : ev) {
+  ~Staging() {
+    for (hipEvent_t e : ev)
       if (e) (void)hipEventDestroy(e);
-      e = nullptr;
-    }
     if (pin) (void)hipHostFree(pin);
-    pin = nullptr;
   }
 };
+
+// The slot sets not in use, kept for the next transfer of any handle of their
+// device (allocating a set takes 2 ms): at most kIdleSets of them, released
+// when the last handle is destroyed.  A transfer owns its set alone.
+class StagingPool {
+ public:
+  static constexpr size_t kIdleSets = 2;
+  void enter() {
+    std::lock_guard<std::mutex> l(mu_);
+    ++handles_;
+  }
+  void leave() {
+    std::unique_ptr<Staging> drop[kIdleSets];
+    std::lock_guard<std::mutex> l(mu_);
+    if (--handles_ == 0)
+      for (size_t q = 0; q < kIdleSets; ++q) drop[q] = std::move(idle_[q]);
+  }
+  std::unique_ptr<Staging> take() {
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess) return nullptr;
+    {
+      std::lock_guard<std::mutex> l(mu_);
+      for (auto& s : idle_)
+        if (s && s->device == dev) return std::move(s);
+    }
+    std::unique_ptr<Staging> s(new (std::nothrow) Staging());
+    if (s && !s->make(dev)) s.reset();
+    return s;
+  }
+  void give(std::unique_ptr<Staging> s) {
+    std::lock_guard<std::mutex> l(mu_);
+    for (auto& q : idle_)
+      if (!q) {
+        q = std::move(s);
+        return;
+      }
+  }
+
+ private:
+  std::mutex mu_;
+  int handles_ = 0;
+  std::unique_ptr<Staging> idle_[kIdleSets];
+};
+// never destroyed: the runtime may be gone by the time static objects are
+inline StagingPool& staging_pool() {
+  static StagingPool* p = new StagingPool();
+  return *p;
+}
 
 // One transfer: chunk c of the segments goes through slot c % kSlots.
 struct Transfer {
@@ -84,8 +125,9 @@ struct Transfer {
   std::atomic<int64_t> moved[kSlots];  // the last chunk whose words a worker moved through the slot, plus one
   std::atomic<bool> stop{false};
 
-  Transfer(const Segment* s, int ns, const Staging& S, bool to_host)
-      : seg(s), nseg(ns), slot(S.slot), pin(S.pin), down(to_host) {
+  Transfer(const Segment* s, int ns, size_t total, const Staging& S, bool to_host)
+      : seg(s), nseg(ns), slot(std::min(kSlotMax, std::max(kSlotMin, total / 16 & ~(size_t)4095))), pin(S.pin),
+        down(to_host) {
     for (int q = 0; q < ns; ++q) n += (int64_t)((s[q].bytes + slot - 1) / slot);
     for (auto& m : moved) m.store(0, std::memory_order_relaxed);
     if (!down) opened.store(kSlots, std::memory_order_relaxed);
@@ -150,11 +192,13 @@ struct Transfer {
 // Copies the segments on `st` and waits for them.  Staged down from 24 MiB and
 // up from 64 MiB; below, and where no slots or threads are to be had, the
 // runtime's copies.
-inline hipError_t transfer(Staging& S, hipStream_t st, const Segment* seg, int nseg, bool to_host) {
+inline hipError_t transfer(hipStream_t st, const Segment* seg, int nseg, bool to_host) {
   size_t total = 0;
   for (int q = 0; q < nseg; ++q) total += seg[q].bytes;
-  if (total >= (to_host ? kStagedDown : kStagedUp) && S.ready(total)) {
-    Transfer T(seg, nseg, S, to_host);
+  std::unique_ptr<Staging> S;
+  if (total >= (to_host ? kStagedDown : kStagedUp)) S = staging_pool().take();
+  if (S) {
+    Transfer T(seg, nseg, total, *S, to_host);
     std::thread th[kWorkers];
     const int want = (int)std::min<int64_t>(std::min<int64_t>(kWorkers, T.n),
                                             std::max(1u, std::thread::hardware_concurrency()));
@@ -164,10 +208,12 @@ inline hipError_t transfer(Staging& S, hipStream_t st, const Segment* seg, int n
     } catch (const std::system_error&) {  // fewer threads share the chunks
     }
     if (have > 0) {
-      const hipError_t e = T.drive(st, S.ev);
+      const hipError_t e = T.drive(st, S->ev);
       for (int t = 0; t < have; ++t) th[t].join();
+      staging_pool().give(std::move(S));
       return e;
     }
+    staging_pool().give(std::move(S));
   }
   for (int q = 0; q < nseg; ++q) {
     const hipError_t e = to_host ? hipMemcpyAsync(seg[q].host, seg[q].dev, seg[q].bytes, hipMemcpyDeviceToHost, st)

@@ -1,4 +1,4 @@
-"""cs_upload_state / cs_download_state through the handle's pinned staging
+"""cs_upload_state / cs_download_state through pinned staging
 slots (down from 24 MiB, up from 64 MiB) and below them: every owned word comes back
 as it went in, whole arrays come back the same from both sizes of call, and a
 download of some of the arrays leaves the others alone."""
