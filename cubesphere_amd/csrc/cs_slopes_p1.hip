@@ -1126,11 +1126,20 @@ __global__ void __launch_bounds__(256) k_zero_hi(const P1 P, const Box b);
 __global__ void __launch_bounds__(64) k_clsq12(const P1 P, const Box b, const double* __restrict__ mom);
 __global__ void __launch_bounds__(256) k_e12(const P1 P, const Box b, const double* __restrict__ mom);
 __global__ void __launch_bounds__(256) k_ao_order(const P1 P, const Box b, unsigned int* bad);
-constexpr int kAoRec = 200;  // doubles per zone record of k_ao_e_pre: G (19 x 10), 18 int32 indices
+constexpr int kAoRec = 208;     // doubles per zone record of k_ao_e_pre
+constexpr int kAoLanes = 16;    // lanes per zone of k_ao_e_sweep
+constexpr int kAoGroups = 28;   // zones of one plane in flight at most (448 threads, and a wave that publishes)
+// the in-plane level of box zone (ir, jr) is ir + s jr: s >= 3 keeps the order,
+// s kAoGroups >= ni leaves at most one row per group of lanes
+__host__ __device__ static inline int ao_stride(int ni) {
+  const int s = (ni + kAoGroups - 1) / kAoGroups;
+  return s < 3 ? 3 : s;
+}
 __global__ void __launch_bounds__(128) k_ao_e_pre(const P1 P, const Box b, const double* __restrict__ mom,
-                                                  double* __restrict__ rec);
-__global__ void __launch_bounds__(64) k_weno_ao_e(const P1 P, const Box b, const double* __restrict__ mom,
-                                                   const double* __restrict__ rec, int level, int klo);
+                                                  double* __restrict__ rec, double* __restrict__ xnew);
+__global__ void __launch_bounds__(kAoLanes * kAoGroups + 64)
+    k_ao_e_sweep(const P1 P, const Box b, double* rec, double* xnew, unsigned int* ticket, int s);
+__global__ void __launch_bounds__(256) k_ao_e_put(const P1 P, const Box b, const double* __restrict__ rec);
 __global__ void __attribute__((amdgpu_waves_per_eu(2))) __launch_bounds__(128)
     k_weno_ao(const P1 P, const Box b, const double* __restrict__ mom, const int64_t* list, int64_t nlist);
 }  // namespace csp1
@@ -1173,7 +1182,7 @@ static int run_p1(const cs_p1_patch* p, void* stream_, float* kernel_ms, uint8_t
   const Box ao = make_box(-1, N + 2, -1, N + 2, -1, NR + 2);
   const size_t base_bytes = (5 * flag_bytes + 256 + (size_t)nblk_diag * 18 * sizeof(double) + 18 * sizeof(double) +
                              list_bytes + 255) / 256 * 256;
-  const size_t need = base_bytes + (mom ? (size_t)ao.count() * kAoRec * sizeof(double) : 0);
+  const size_t need = base_bytes + (mom ? (size_t)ao.count() * (kAoRec + 4) * sizeof(double) : 0);
   if (mom && P.NZ >= ((int64_t)1 << 31)) {
     cs::set_error("cs_limit_all_slopes_p12: the patch has %lld zones, more than int32 indices reach",
                   (long long)P.NZ);
@@ -1328,19 +1337,16 @@ static int run_p1(const cs_p1_patch* p, void* stream_, float* kernel_ms, uint8_t
   if ((rc = mark())) return rc;
   k_weno9<<<grid_of(wr.count(), 128), 128, 0, st>>>(P, wr, nullptr, 0, we);
   if (mom) {
-    // 9.c in the loop order of the reference's serial build: level
-    // (i+1) + 3 (j+1) + 9 (k+1) of the zone box; k_ao_order flags a stencil
-    // table for which a zone's earlier neighbours are not all on lower
-    // levels and its later ones all on higher levels
-    P1_HIP(hipMemsetAsync(F.counter + 2, 0, sizeof(unsigned int), st));
+    // 9.c in the loop order of the reference's serial build (k_ao_e_sweep);
+    // k_ao_order flags a stencil table for which a zone's earlier neighbours
+    // are not all on lower levels and its later ones all on higher levels
+    double* xnew = aorec + (size_t)ao.count() * kAoRec;
+    const int sj = ao_stride(ao.ni), threads = ((ao.ni + sj - 1) / sj * kAoLanes + 63) / 64 * 64 + 64;
+    P1_HIP(hipMemsetAsync(F.counter + 2, 0, 2 * sizeof(unsigned int), st));
     k_ao_order<<<grid_of((int64_t)ao.ni * ao.nj, 256), 256, 0, st>>>(P, ao, F.counter + 2);
-    k_ao_e_pre<<<grid_of(ao.count(), 128), 128, 0, st>>>(P, ao, mom, aorec);
-    const int top = (ao.ni - 1) + 3 * (ao.nj - 1) + 9 * (ao.nk - 1);
-    for (int lv = 0; lv <= top; ++lv) {
-      const int klo = std::max(0, (lv - (ao.ni - 1) - 3 * (ao.nj - 1) + 8) / 9);
-      const int khi = std::min(ao.nk - 1, lv / 9);
-      k_weno_ao_e<<<grid_of(3 * (int64_t)ao.nj * (khi - klo + 1), 64), 64, 0, st>>>(P, ao, mom, aorec, lv, klo);
-    }
+    k_ao_e_pre<<<grid_of(ao.count(), 128), 128, 0, st>>>(P, ao, mom, aorec, xnew);
+    k_ao_e_sweep<<<ao.nk, threads, 0, st>>>(P, ao, aorec, xnew, F.counter + 3, sj);
+    k_ao_e_put<<<grid_of(ao.count(), 256), 256, 0, st>>>(P, ao, aorec);
   }
   if ((rc = mark())) return rc;
   k_diag<<<nblk_diag, DIAG_THREADS, 0, st>>>(P, all, part);
@@ -3249,26 +3255,44 @@ __global__ void __launch_bounds__(256) k_ao_order(const P1 P, const Box b, unsig
 // of E only through its right-hand side: the ten modes are X = G R, R the 19
 // point values, G = (A^T A)^-1 A^T, A the 19 x 10 matrix of
 // INTERPOLATION_COEFS (252interpolation_coefs.f:5: this zone's basis at each
-// stencil zone's centroid, row 0 the zone itself).  k_ao_e_pre forms G for
-// every active zone of the box, one thread per zone, with a Cholesky factor
-// of A^T A, and stores it with the 18 stencil zones' indices as one record of
-// kAoRec doubles per zone (G row-major by stencil row, then the indices as
-// int32), so that the ordered sweep reads one contiguous record per zone.
+// stencil zone's centroid, row 0 the zone itself).  k_ao_e_pre, one thread
+// per zone of the box, forms G with a Cholesky factor of A^T A, adds up the
+// part of X that the loop order leaves at old point values (the zone itself,
+// the zones after it and the inactive ones), and keeps, as one record of
+// kAoRec doubles, what the ordered sweep needs: G's rows for the zones of the
+// plane below and for the earlier zones of the same plane, that partial sum,
+// and the zone's own terms of the hybridisation.  Doubles of a record:
+constexpr int kAoG = 0;      // [10 modes][10]: G for the five zones below, then for the first four earlier zones of
+                             // the plane
+constexpr int kAoOut = 0;    // [10][4] in their place, after the sweep: the zone's new modes of E
+constexpr int kAoPo = 100;   // [10][4]: the old values' part of X for the three components, the smoothness
+                             // indicator's weight of the mode
+constexpr int kAoEe = 140;   // [4][4]: the point value and the WENO gradient of the three components of E
+constexpr int kAoMi = 156;   // [4]: the three low indicators, the flattener
+constexpr int kAoIx = 160;   // 16 int32: [0..4] box index of each zone below (-1: none), [5] how many earlier zones of
+                             // the plane (-1: an inactive zone), [8..15] these (ring slot, or -2 - box index)
+constexpr int kAoGf = 168;   // [4][10]: G for further earlier zones (tri-corner strips)
+// the newest values of each row of a plane in LDS: rows modulo kRingRows, the
+// last kRing zones of a row
+constexpr int kRing = 16, kRingRows = 64;
+// no result of arithmetic: a signalling NaN marks a point value not yet formed
+constexpr unsigned long long kAoEmpty = 0x7ff0dead0badf00dull;
 
 __global__ void __launch_bounds__(128) k_ao_e_pre(const P1 P, const Box b, const double* __restrict__ mom,
-                                                  double* __restrict__ rec) {
+                                                  double* __restrict__ rec, double* __restrict__ xnew) {
   const int64_t t = tid();
   int i, j, k;
   if (!b.decode(t, i, j, k)) return;
   const cs_p1_patch& a = P.a;
   const int64_t z = P.zi(i, j, k), NZ = P.NZ;
-  if (!P.active(i, j, 1)) {  // the sweep loads an inactive zone's stencil too, and discards it
-    int* idx = (int*)(rec + t * kAoRec + 190);
 #pragma unroll
-    for (int r = 0; r < 18; ++r) idx[r] = (int)z;
+  for (int c = 0; c < 3; ++c) ((unsigned long long*)xnew)[4 * t + c] = kAoEmpty;
+  if (!P.active(i, j, 1)) {  // the sweep skips it
+    ((int*)(rec + t * kAoRec + kAoIx))[5] = -1;
     return;
   }
-  const double obl0 = 1.0 / fmax(a.scale[z], a.smallnum);
+  const double sm = a.smallnum;
+  const double obl0 = 1.0 / fmax(a.scale[z], sm);
   double c0[6], cz[3];
 #pragma unroll
   for (int m = 0; m < 6; ++m) c0[m] = mom[z + NZ * (4 + m)];
@@ -3281,18 +3305,12 @@ __global__ void __launch_bounds__(128) k_ao_e_pre(const P1 P, const Box b, const
     for (int q = 0; q < 8; ++q) P.nbr(i, j, dirs[q], ni[q], nj[q]);
   }
   double* G = rec + t * kAoRec;
-  int* idx = (int*)(G + 190);
+  int* ix = (int*)(G + kAoIx);
   // row r of A: r = 0 the zone itself, r = 1..18 the stencil zones
-  auto arow = [&](int r, double* row) {
-    if (r == 0) {
-      row[0] = 1.0;
-      row[1] = row[2] = row[3] = 0.0;
-#pragma unroll
-      for (int m = 0; m < 6; ++m) row[4 + m] = -c0[m];
-      return;
-    }
+  auto where = [&](int r, int& ii, int& jj) {
     const int dir = c_ao_dir[r - 1];
-    int ii = i, jj = j;
+    ii = i;
+    jj = j;
     if (dir >= 0) {
 #pragma unroll
       for (int q = 0; q < 8; ++q)
@@ -3301,7 +3319,15 @@ __global__ void __launch_bounds__(128) k_ao_e_pre(const P1 P, const Box b, const
           jj = nj[q];
         }
     }
-    const int64_t zr = P.zi(ii, jj, k + c_ao_dk[r - 1]);
+  };
+  auto arow = [&](int r, int64_t zr, double* row) {
+    if (r == 0) {
+      row[0] = 1.0;
+      row[1] = row[2] = row[3] = 0.0;
+#pragma unroll
+      for (int m = 0; m < 6; ++m) row[4 + m] = -c0[m];
+      return;
+    }
     double x[3];
 #pragma unroll
     for (int c = 0; c < 3; ++c) x[c] = (a.v_centroid[zr + NZ * c] - cz[c]) * obl0;
@@ -3315,7 +3341,6 @@ __global__ void __launch_bounds__(128) k_ao_e_pre(const P1 P, const Box b, const
     row[7] = x[0] * x[1] - c0[3];
     row[8] = x[1] * x[2] - c0[4];
     row[9] = x[0] * x[2] - c0[5];
-    idx[r - 1] = (int)zr;
   };
   double L[55];
 #pragma unroll
@@ -3323,7 +3348,12 @@ __global__ void __launch_bounds__(128) k_ao_e_pre(const P1 P, const Box b, const
 #pragma unroll 1
   for (int r = 0; r < 19; ++r) {
     double row[10];
-    arow(r, row);
+    int ii = i, jj = j, dk = 0;
+    if (r > 0) {
+      where(r, ii, jj);
+      dk = c_ao_dk[r - 1];
+    }
+    arow(r, P.zi(ii, jj, k + dk), row);
 #pragma unroll
     for (int p = 0; p < 10; ++p)
 #pragma unroll
@@ -3346,10 +3376,23 @@ __global__ void __launch_bounds__(128) k_ao_e_pre(const P1 P, const Box b, const
       L[r * (r + 1) / 2 + p] = t2 * od[p];
     }
   }
+  double po[3][10];
+#pragma unroll
+  for (int c = 0; c < 3; ++c)
+#pragma unroll
+    for (int m = 0; m < 10; ++m) po[c][m] = 0.0;
+  const int s = ao_stride(b.ni);
+  int nb = 0, nn = 0;
 #pragma unroll 1
   for (int r = 0; r < 19; ++r) {  // column r of G: (A^T A)^-1 times row r
+    int ii = i, jj = j, dk = 0;
+    if (r > 0) {
+      where(r, ii, jj);
+      dk = c_ao_dk[r - 1];
+    }
+    const int64_t zr = P.zi(ii, jj, k + dk);
     double X[10];
-    arow(r, X);
+    arow(r, zr, X);
 #pragma unroll
     for (int p = 0; p < 10; ++p) {
       double t2 = X[p];
@@ -3364,87 +3407,339 @@ __global__ void __launch_bounds__(128) k_ao_e_pre(const P1 P, const Box b, const
       for (int q = p + 1; q < 10; ++q) t2 -= L[q * (q + 1) / 2 + p] * X[q];
       X[p] = t2 * od[p];
     }
+    // the zone's new value is read if the serial loop has passed it: an
+    // active zone of the box in the plane below, or earlier in this one
+    const int di = ii - i, dj = jj - j, back = -(di + s * dj);
+    const bool in = ii >= b.i0 && ii < b.i0 + b.ni && jj >= b.j0 && jj < b.j0 + b.nj && k + dk >= b.k0 &&
+                    k + dk < b.k0 + b.nk && P.active(ii, jj, 1);
+    const int bi = (ii - b.i0) + b.ni * ((jj - b.j0) + b.nj * (k + dk - b.k0));
+    int col = -1;
+    double* far = nullptr;
+    if (in && dk < 0) {
+      ix[nb] = bi;
+      col = nb++;
+    } else if (in && dk == 0 && (dj < 0 || (dj == 0 && di < 0)) && back > 0) {
+      ix[8 + nn] = back < kRing ? ((jj - b.j0) % kRingRows) * kRing + (ii - b.i0) % kRing : -2 - bi;
+      if (nn < 4) col = 5 + nn;
+      else far = G + kAoGf + 10 * (nn - 4);
+      ++nn;
+    }
+    if (col >= 0) {
 #pragma unroll
-    for (int m = 0; m < 10; ++m) G[10 * r + m] = X[m];
+      for (int m = 0; m < 10; ++m) G[kAoG + 10 * m + col] = X[m];
+    } else if (far) {
+#pragma unroll
+      for (int m = 0; m < 10; ++m) far[m] = X[m];
+    } else {
+      const double E[3] = {a.Ex_zc[zr], a.Ey_zc[zr], a.Ez_zc[zr]};
+#pragma unroll
+      for (int c = 0; c < 3; ++c)
+#pragma unroll
+        for (int m = 0; m < 10; ++m) po[c][m] += X[m] * E[c];
+    }
   }
-}
-
-// Step 9.c at third order (421...f:8406-9353) for component c of E at box
-// zone (ir, jr, kr): the ten modes of the quadratic interpolant X = G R from
-// the zone's record (k_ao_e_pre) and the point values of E at the zone and
-// its 18 stencil zones; the hybridisation with the WENO gradients of 9.b as
-// in 7.b, then the point value E_pt f + E (1 - f) and the modes times (1 - f).
-__device__ __forceinline__ void ao_e_zone(const P1& P, const Box& b, const double* __restrict__ mom,
-                                          const double* __restrict__ rec, int ir, int jr, int kr, int c) {
-  const int i = b.i0 + ir, j = b.j0 + jr, k = b.k0 + kr;
-  const cs_p1_patch& a = P.a;
-  // the loads go out before the mask is known: an inactive zone's record
-  // points at the zone itself, and only an active zone writes
-  const int64_t z = P.zi(i, j, k), NZ = P.NZ;
-  const bool act = P.active(i, j, 1);
-  const double* G = rec + ((int64_t)ir + (int64_t)b.ni * (jr + (int64_t)b.nj * kr)) * kAoRec;
-  const int* idx = (const int*)(G + 190);
-  double* E = c == 0 ? a.Ex_zc : (c == 1 ? a.Ey_zc : a.Ez_zc);
-  double X[10];
-  const double Ept = E[z];
+  for (int q = nb; q < 5; ++q) {
+    ix[q] = -1;
 #pragma unroll
-  for (int m = 0; m < 10; ++m) X[m] = G[m] * Ept;
-#pragma unroll
-  for (int r = 1; r < 19; ++r) {
-    const double R = E[idx[r - 1]];
-#pragma unroll
-    for (int m = 0; m < 10; ++m) X[m] += G[10 * r + m] * R;
+    for (int m = 0; m < 10; ++m) G[kAoG + 10 * m + q] = 0.0;
   }
-  double c0[6];
-#pragma unroll
-  for (int m = 0; m < 6; ++m) c0[m] = mom[z + NZ * (4 + m)];
-  const double sm = a.smallnum, f = a.flatten[z];
-  const double betalo = f + (1.0 - f) * 2.0;
-  const double gammahi = f * 0.6 + (1.0 - f) * 0.95, gammalo = 1.0 - gammahi;
-  const double obgammahi = 1.0 / gammahi, gammaratio = gammalo / gammahi;
-  const double ob12 = 1.0 / 12.0, ob180 = 1.0 / 180.0, ob144 = 1.0 / 144.0;
+  ix[5] = nn;
+  // the zone's own terms (421...f:8937-9030)
+  const double ob12 = 1.0 / 12.0, ob180 = 1.0 / 180.0, ob144 = 1.0 / 144.0, f = a.flatten[z];
   const double m5 = c0[0] - ob12, m6 = c0[1] - ob12, m7 = c0[2] - ob12;
-  double e[4];
+  const double wt[10] = {0.0, ob12, ob12, ob12, m5 * m5 + ob180, m6 * m6 + ob180, m7 * m7 + ob180,
+                         c0[3] * c0[3] + ob144, c0[4] * c0[4] + ob144, c0[5] * c0[5] + ob144};
 #pragma unroll
-  for (int m = 0; m < 4; ++m) e[m] = E[z + NZ * m];
-  const double ISlo = betalo * (e[1] * e[1] + e[2] * e[2] + e[3] * e[3]) * ob12;
-  double Phi[10];
+  for (int m = 0; m < 10; ++m) {
 #pragma unroll
-  for (int m = 0; m < 4; ++m) Phi[m] = X[m] * obgammahi - e[m] * gammaratio;
+    for (int c = 0; c < 3; ++c) G[kAoPo + 4 * m + c] = po[c][m];
+    G[kAoPo + 4 * m + 3] = wt[m];
+  }
+  const double betalo = f + (1.0 - f) * 2.0;
 #pragma unroll
-  for (int m = 4; m < 10; ++m) Phi[m] = X[m] * obgammahi;
-  const double IShi = (Phi[1] * Phi[1] + Phi[2] * Phi[2] + Phi[3] * Phi[3]) * ob12 +
-                      Phi[4] * Phi[4] * (m5 * m5 + ob180) + Phi[5] * Phi[5] * (m6 * m6 + ob180) +
-                      Phi[6] * Phi[6] * (m7 * m7 + ob180) + Phi[7] * Phi[7] * (c0[3] * c0[3] + ob144) +
-                      Phi[8] * Phi[8] * (c0[4] * c0[4] + ob144) + Phi[9] * Phi[9] * (c0[5] * c0[5] + ob144);
-  const double tau = fabs(IShi - ISlo);
-  double wlo = gammalo * (1.0 + tau / (ISlo + sm)), whi = gammahi * (1.0 + tau / (IShi + sm));
-  const double aa = 1.0 / (wlo + whi);
-  wlo *= aa;
-  whi *= aa;
-  const double x1 = 1.0 - f;
-  if (!act) return;
-  E[z] = Ept * f + (whi * Phi[0] + wlo * e[0]) * x1;
+  for (int c = 0; c < 3; ++c) {
+    const double* E = c == 0 ? a.Ex_zc : (c == 1 ? a.Ey_zc : a.Ez_zc);
+    double e[4];
 #pragma unroll
-  for (int m = 1; m < 4; ++m) E[z + NZ * m] = (whi * Phi[m] + wlo * e[m]) * x1;
-#pragma unroll
-  for (int m = 4; m < 10; ++m) E[z + NZ * m] = whi * Phi[m] * x1;
+    for (int m = 0; m < 4; ++m) {
+      e[m] = E[z + NZ * m];
+      G[kAoEe + 4 * m + c] = e[m];
+    }
+    G[kAoMi + c] = betalo * (e[1] * e[1] + e[2] * e[2] + e[3] * e[3]) * ob12;
+  }
+  G[kAoMi + 3] = f;
 }
 
-// Step 9.c in the serial loop order (k_ao_order): one launch per level
-// (i+1) + 3 (j+1) + 9 (k+1) of the box, three lanes per zone (one per
-// component of E), the box's (j, k) rows from plane klo on.  The zones of a
-// level read none of each other; the launches order the levels.
-__global__ void __launch_bounds__(64) k_weno_ao_e(const P1 P, const Box b, const double* __restrict__ mom,
-                                                   const double* __restrict__ rec, int level, int klo) {
-  const int64_t t = tid();
-  const int c = (int)(t % 3);
-  const int64_t tz = t / 3;
-  const int jr = (int)(tz % b.nj), kr = klo + (int)(tz / b.nj);
+// the sum over a row of 16 lanes, in every lane: neighbours, pairs, then the
+// mirror images within eight and sixteen lanes
+template <int CTRL>
+__device__ __forceinline__ double dpp_add(double v) {
+  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, 0xf, 0xf, true);
+  return v + __hiloint2double(hi, lo);
+}
+__device__ __forceinline__ double row_sum(double v) {
+  v = dpp_add<0xb1>(v);       // quad_perm 1 0 3 2
+  v = dpp_add<0x4e>(v);       // quad_perm 2 3 0 1
+  v = dpp_add<0x141>(v);      // row_half_mirror
+  return dpp_add<0x140>(v);   // row_mirror
+}
+// LDS words written before by a wave's lanes, read after by its others
+__device__ __forceinline__ void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+// The workgroup's waves meet with their LDS words written and read.  Only the
+// ring passes between the waves of a plane, so nothing waits for the stores to
+// memory (a full barrier would, and a store's acknowledgement takes longer
+// than a level's arithmetic).
+__device__ __forceinline__ void ring_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+__device__ __forceinline__ double ao_load(const double* p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ bool ao_empty(double v) { return (unsigned long long)__double_as_longlong(v) == kAoEmpty; }
+
+// Step 9.c at third order (421...f:8406-9353) in the serial loop order: the
+// ten modes of the quadratic interpolant X = G R, their hybridisation with
+// the WENO gradients of 9.b as in 7.b, then the point value
+// E_pt f + E (1 - f) and the modes times (1 - f).
+//
+// One workgroup per plane k of the box walks the in-plane levels
+// l = ir + s jr; a group of 16 lanes takes the zone of its row (rows
+// jr = group, group + Z, ...; Z s >= ni, so a group has one row at a time),
+// lane m < 10 the mode m of the three components, so that no lane loads what
+// another has (a quad of lanes per component loaded G three times and was
+// bound by the address unit).  A zone's record and the values of the plane
+// below are read two levels ahead, its indices three; the values of the same
+// plane, written in the last levels, come from a ring of the newest values of
+// each row in LDS (a tri-corner zone's entry further back from memory), so
+// the chain of a level is: ring, four rows of G, the sum of the indicator
+// over the group, the weights, ring.
+//
+// The planes run side by side.  A point value leaves its plane through xnew
+// (device-scope relaxed stores and loads of 8 bytes; old values stay in E
+// until k_ao_e_put), and the value itself says that it is there (kAoEmpty
+// until then), so nothing needs fences, and a plane follows the one below a
+// few levels behind.  Planes are handed out by a ticket in the order that
+// workgroups start: a workgroup waits only for the plane of the previous
+// ticket, which a running or finished workgroup has, and within its own plane
+// only for levels it has passed, so every wait ends, whatever the table.
+//
+// What bounds it: the chain of (ni - 1) + s (nj - 1) levels and a lag of some
+// ten levels a plane, 2 to 3 us a level (the latency of the zone's own loads
+// and of the values below, the arithmetic of one wave).  Step 9 with the
+// pre-pass, against one launch per level of all planes (9 to 13 us each):
+// 64^2 x 25 5.0 -> 1.5 ms (521 launches), 192^2 x 64 20.6 -> 11.9 ms (1,384).
+__global__ void __launch_bounds__(kAoLanes * kAoGroups + 64)
+    k_ao_e_sweep(const P1 P, const Box b, double* rec, double* xnew, unsigned int* ticket, int s) {
+  __shared__ double2 ringv[kRingRows * kRing][2];   // the three components of a point value
+  __shared__ double2 upv[kAoGroups][8];             // a group's values of the plane below, [zone][component]
+  __shared__ int2 pub[2][kAoGroups];                // a level's zones: ring slot, box index (-1: none)
+  __shared__ int plane;
+  if (threadIdx.x == 0) plane = (int)atomicAdd(ticket, 1u);
+  __syncthreads();
+  const int kr = plane;
   if (kr >= b.nk) return;
-  const int ir = level - 3 * jr - 9 * kr;
-  if (ir < 0 || ir >= b.ni) return;
-  ao_e_zone(P, b, mom, rec, ir, jr, kr, c);
+  const double sm = P.a.smallnum;
+  const int Z = (blockDim.x - 64) / kAoLanes, g = threadIdx.x / kAoLanes, ln = threadIdx.x % kAoLanes;
+  const int m = ln < 10 ? ln : 9;  // lanes 10 to 15 repeat mode 9 with weight 0
+  const int ur = ln < 15 ? ln / 3 : 4, uc = ln < 15 ? ln % 3 : 2;  // the value below that this lane reads
+  const int levels = b.ni + s * (b.nj - 1);
+  struct Index {
+    int4 near;
+    int nn, below, ir, jr;
+    bool on;
+  };
+  struct Zone {
+    Index x;
+    double2 G[5], p01, p2w, e01, e2, i01, i2f;
+    double acc[3], up;
+  };
+  auto box_index = [&](int ir, int jr) { return ir + (int64_t)b.ni * (jr + (int64_t)b.nj * kr); };
+  if (g >= Z) {
+    // the last wave sends each level's point values on after the level: a
+    // store's acknowledgement counts before the loads that a wave put out
+    // after it, so the waves that form the values send none
+    for (int l = 0; l < (levels + 2) / 3 * 3; ++l) {
+      ring_barrier();
+      for (int e = threadIdx.x % 64; e < 3 * Z; e += 64) {
+        const int2 w = pub[l & 1][e / 3];
+        if (w.y >= 0)
+          __hip_atomic_store(xnew + 4 * (int64_t)w.y + e % 3, ((const double*)ringv[w.x])[e % 3], __ATOMIC_RELAXED,
+                             __HIP_MEMORY_SCOPE_AGENT);
+      }
+    }
+    return;
+  }
+  // group g's zone of level l: its row, if it has one there, and the indices
+  // of its record
+  auto place = [&](int l, Index& I) {
+    const int jmax = l / s;
+    I.on = false;
+    if (l >= levels || jmax < g) return;
+    I.jr = jmax - (jmax - g) % Z;
+    I.ir = l - s * I.jr;
+    if (I.jr >= b.nj || I.ir >= b.ni) return;
+    I.on = true;
+    const int* ix = (const int*)(rec + box_index(I.ir, I.jr) * kAoRec + kAoIx);
+    I.below = ix[ur];
+    I.nn = ix[5];
+    I.near = *(const int4*)(ix + 8);
+  };
+  // the loads of the zone's record and of its values below go out
+  auto issue = [&](const Index& I, Zone& Q) {
+    Q.x = I;
+    Q.x.on = I.on && I.nn >= 0;
+    if (!Q.x.on) return;
+    Q.up = 0.0;
+    if (I.below >= 0) Q.up = ao_load(xnew + 4 * (int64_t)I.below + uc);
+    const double* R = rec + box_index(I.ir, I.jr) * kAoRec;
+    const double2* g2 = (const double2*)(R + kAoG + 10 * m);
+#pragma unroll
+    for (int r = 0; r < 5; ++r) Q.G[r] = g2[r];
+    const double2* p2 = (const double2*)(R + kAoPo + 4 * m);
+    Q.p01 = p2[0];
+    Q.p2w = p2[1];
+    const double2* e2 = (const double2*)(R + kAoEe + 4 * (m < 4 ? m : 0));
+    Q.e01 = e2[0];
+    Q.e2 = e2[1];
+    const double2* i2 = (const double2*)(R + kAoMi);
+    Q.i01 = i2[0];
+    Q.i2f = i2[1];
+  };
+  auto add = [&](Zone& Q, double gv, double2 v01, double v2) {
+    Q.acc[0] += gv * v01.x;
+    Q.acc[1] += gv * v01.y;
+    Q.acc[2] += gv * v2;
+  };
+  // the plane below's values arrive and enter the sum
+  auto settle = [&](Zone& Q) {
+    if (!Q.x.on) return;
+    while (ao_empty(Q.up)) {
+      __builtin_amdgcn_s_sleep(1);
+      Q.up = ao_load(xnew + 4 * (int64_t)Q.x.below + uc);
+    }
+    ((double*)upv[g])[ln] = Q.up;
+    wave_sync();
+    Q.acc[0] = Q.p01.x;
+    Q.acc[1] = Q.p01.y;
+    Q.acc[2] = Q.p2w.x;
+    double2 u[8];
+#pragma unroll
+    for (int r = 0; r < 8; ++r) u[r] = upv[g][r];
+    add(Q, Q.G[0].x, u[0], u[1].x);
+    add(Q, Q.G[0].y, make_double2(u[1].y, u[2].x), u[2].y);
+    add(Q, Q.G[1].x, u[3], u[4].x);
+    add(Q, Q.G[1].y, make_double2(u[4].y, u[5].x), u[5].y);
+    add(Q, Q.G[2].x, u[6], u[7].x);
+    wave_sync();
+  };
+  auto newest = [&](Zone& Q, int code, double gv) {
+    if (code >= 0) {
+      add(Q, gv, ringv[code][0], ringv[code][1].x);
+    } else {
+      double v[3];
+#pragma unroll
+      for (int c = 0; c < 3; ++c) {
+        const double* p = xnew + 4 * (int64_t)(-2 - code) + c;
+        v[c] = ao_load(p);
+        while (ao_empty(v[c])) v[c] = ao_load(p);
+      }
+      add(Q, gv, make_double2(v[0], v[1]), v[2]);
+    }
+  };
+  auto form = [&](Zone& Q, int l) {
+    if (!Q.x.on) {
+      if (ln == 0) pub[l & 1][g].y = -1;
+      return;
+    }
+    if (Q.x.nn > 0) newest(Q, Q.x.near.x, Q.G[2].y);
+    if (Q.x.nn > 1) newest(Q, Q.x.near.y, Q.G[3].x);
+    if (Q.x.nn > 2) newest(Q, Q.x.near.z, Q.G[3].y);
+    if (Q.x.nn > 3) newest(Q, Q.x.near.w, Q.G[4].x);
+    const int64_t t = box_index(Q.x.ir, Q.x.jr);
+    for (int r = 4; r < Q.x.nn; ++r) {  // tri-corner strips only
+      const double* R = rec + t * kAoRec;
+      newest(Q, ((const int*)(R + kAoIx))[8 + r], R[kAoGf + 10 * (r - 4) + m]);
+    }
+    const double f = Q.i2f.y, x1 = 1.0 - f, gh = f * 0.6 + x1 * 0.95, gl = 1.0 - gh;
+    const double obg = 1.0 / gh, gr = gl / gh;
+    const double e[3] = {ln < 4 ? Q.e01.x : 0.0, ln < 4 ? Q.e01.y : 0.0, ln < 4 ? Q.e2.x : 0.0};
+    const double lo[3] = {Q.i01.x, Q.i01.y, Q.i2f.x};
+    const double w = ln < 10 ? Q.p2w.y : 0.0;
+    double o[3];
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+      const double p = Q.acc[c] * obg - e[c] * gr, hi = row_sum(p * p * w), tau = fabs(hi - lo[c]);
+      const double wlo = gl * (1.0 + tau / (lo[c] + sm)), whi = gh * (1.0 + tau / (hi + sm));
+      const double aa = 1.0 / (wlo + whi);
+      o[c] = (whi * aa * p + wlo * aa * e[c]) * x1;
+    }
+    if (ln == 0) {  // the point value
+#pragma unroll
+      for (int c = 0; c < 3; ++c) o[c] = e[c] * f + o[c];
+      const int slot = (Q.x.jr % kRingRows) * kRing + Q.x.ir % kRing;
+      ringv[slot][0] = make_double2(o[0], o[1]);
+      ringv[slot][1].x = o[2];
+      pub[l & 1][g] = make_int2(slot, (int)t);
+    }
+    if (ln < 10) {  // the modes take the place of the rows that have been read
+      double2* v = (double2*)(rec + t * kAoRec + kAoOut + 4 * ln);
+      v[0] = make_double2(o[0], o[1]);
+      v[1].x = o[2];
+    }
+  };
+  // three zones in turn: at level l, l + 2's loads go out, l's values are
+  // formed and l + 1's loads, put out a level ago, are waited for
+  Zone A, B, C;
+  Index ia, ib, ic;
+  place(0, ia);
+  place(1, ib);
+  place(2, ic);
+  issue(ia, A);
+  issue(ib, B);
+  settle(A);
+#pragma unroll 1
+  for (int l = 0; l < levels; l += 3) {
+    place(l + 3, ia);
+    issue(ic, C);
+    form(A, l);
+    settle(B);
+    ring_barrier();
+    place(l + 4, ib);
+    issue(ia, A);
+    form(B, l + 1);
+    settle(C);
+    ring_barrier();
+    place(l + 5, ic);
+    issue(ib, B);
+    form(C, l + 2);
+    settle(A);
+    ring_barrier();
+  }
+}
+
+// the active zones' modes from their records into E, once no zone reads the
+// old point values: the sweep's own stores then stay within a zone's record
+// (30 words together) instead of 30 places far apart
+__global__ void __launch_bounds__(256) k_ao_e_put(const P1 P, const Box b, const double* __restrict__ rec) {
+  const int64_t t = tid();
+  int i, j, k;
+  if (!b.decode(t, i, j, k) || !P.active(i, j, 1)) return;
+  const int64_t z = P.zi(i, j, k);
+  const double2* R = (const double2*)(rec + t * kAoRec + kAoOut);
+#pragma unroll
+  for (int m = 0; m < 10; ++m) {
+    const double2 v = R[2 * m];
+    P.a.Ex_zc[z + P.NZ * m] = v.x;
+    P.a.Ey_zc[z + P.NZ * m] = v.y;
+    P.a.Ez_zc[z + P.NZ * m] = R[2 * m + 1].x;
+  }
 }
 
 }  // namespace csp1

@@ -44,6 +44,9 @@ CASES = [
     (8, 3, 3, 9, True, 0.6, 5),  # NGhost 5
     (5, 2, 0, 11, True, 0.8),  # a patch barely wider than its ghosts
     (9, 3, 4, 13, False, 0.3),  # odd N
+    # step 9.c's sweep beyond three levels a row (92 zones across) and past the 64 rows of its ring; a thin
+    # shell, so that the zones are not 30 times deeper than wide
+    (88, 1, 2, 21, True, 0.3, 4, 1.02),
 ]
 
 
@@ -64,7 +67,8 @@ def test_p12_zones_match_oracle(case):
     N, NR, s, seed, shock, noise = case[:6]
     g = case[6] if len(case) > 6 else 4
     print(f"case p12 zones {case}", flush=True)
-    prob, A0 = orc.p12_problem(N, NR, g, sector=s, seed=seed, shock=shock, noise=noise)
+    kw = dict(rmax=case[7]) if len(case) > 7 else {}
+    prob, A0 = orc.p12_problem(N, NR, g, sector=s, seed=seed, shock=shock, noise=noise, **kw)
     O = orc.p12_oracle(prob, orc.p1_copy(A0))
     G = _run_gpu(prob, orc.p1_copy(A0))
     nz = orc.p1_dims(N, NR, g)["zone"]
