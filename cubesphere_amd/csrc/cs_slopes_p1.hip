@@ -30,12 +30,12 @@
 // later zones of the loop then see in their entropy range.  k_pos runs all
 // zones with the incoming entropy means and flags the zones that fail
 // completely; when any do, the zones with such a neighbour earlier in the
-// loop order (k_cands) are recomputed (k_weno9, k_pos on that list) with the
-// means of the flagged earlier zones taken as zero, repeating until the flags
-// no longer change; a zone flagged for the first time in a sweep brings its
-// later neighbours onto the list before the next sweep (the dependence only
-// runs forward in the loop order, so this reaches the sequential result), and
-// the flagged means are then cleared.
+// loop order (k_cands) are recomputed (k_replay) with the means of the flagged
+// earlier zones taken as zero, repeating until the flags no longer change; a
+// zone flagged for the first time in a sweep brings its later neighbours onto
+// the list before the next sweep (the dependence only runs forward in the
+// loop order, so this reaches the sequential result), and the flagged means
+// are then cleared.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -108,12 +108,41 @@ static Box make_box(int i0, int i1, int j0, int j1, int k0, int k1) {
 __device__ __forceinline__ int64_t tid() { return (int64_t)blockIdx.x * blockDim.x + threadIdx.x; }
 
 // ---------------------------------------------------------------------------
+// step 7.b, the positivity limiter (pos_zone)
+// sweep < 0: every zone of the range with the incoming entropy means; sets its
+// flags and counts the zones whose slopes were removed.
+// sweep >= 0: a zone of the replay list (those with a flagged zone earlier in
+// the loop order among their 27), taking the entropy means of the earlier
+// zones flagged by the sweep before as zero; sets its flag for the next sweep
+// and counts the zones whose flag changed.
+constexpr int kMaxSweeps = 256;  // the replay has to settle within these
+constexpr int kSweepBatch = 4;   // sweeps put on the stream between two looks of the host
+struct Flags {
+  uint8_t* fl[2];          // [zone]: sweep n reads fl[n % 2] and writes fl[(n + 1) % 2]
+  uint8_t *ever, *inlist;  // [zone]: flagged in the first pass or any sweep; on the list
+  int64_t* list;
+  // [0] zones whose slopes the first pass removed, [1] list length, [2] and
+  // [3] of step 9.c, [4 + n] flag changes of sweep n
+  unsigned int* ctr;
+  // a sweep after one that changed no flag has nothing to do; its own change
+  // count, zero from the start, passes that on
+  __device__ __forceinline__ bool done(int sweep) const {
+    return ctr[0] == 0 || (sweep > 0 && ctr[4 + sweep - 1] == 0);
+  }
+};
+constexpr int kCtrWords = 4 + kMaxSweeps;
+
+// ---------------------------------------------------------------------------
 // steps 2 and 5
-__global__ void __launch_bounds__(256) k_prim(const P1 P, const Box b) {
+// and the positivity limiter's flags and counters start clear
+__global__ void __launch_bounds__(256) k_prim(const P1 P, const Box b, const Flags F) {
   int i, j, k;
+  if (blockIdx.x == 0)
+    for (int q = threadIdx.x; q < kCtrWords; q += blockDim.x) F.ctr[q] = 0;
   if (!b.decode(tid(), i, j, k)) return;
   const cs_p1_patch& a = P.a;
   const int64_t z = P.zi(i, j, k);
+  F.fl[0][z] = F.fl[1][z] = F.ever[z] = F.inlist[z] = 0;
   const double gam = a.gamma;
   a.gamma_eos[z] = gam;
   a.gamma_sound[z] = gam;
@@ -347,22 +376,7 @@ struct WenoFields {
 // added at the end and the sum normalised.  The stencil's neighbours are
 // chosen by selects: indexing the small arrays by the loop counter would put
 // them in scratch.
-__global__ void __launch_bounds__(128) k_weno9(const P1 P, const Box b, const int64_t* list, int64_t nlist,
-                                               const WenoFields W9) {
-  // thread t: fields 3 (t / n) .. 3 (t / n) + 2 of zone t % n
-  const int64_t t = tid(), n = list ? nlist : b.count();
-  const int ngroups = (W9.n + 2) / 3;
-  if (t >= ngroups * n) return;
-  const int c0 = 3 * (int)(t / n);
-  int i, j, k;
-  int64_t z;
-  if (list) {
-    z = list[t % n];
-    zone_of(P, z, i, j, k);
-  } else {
-    b.decode(t % n, i, j, k);
-    z = P.zi(i, j, k);
-  }
+__device__ __forceinline__ void weno_group(const P1& P, int i, int j, int k, int64_t z, int c0, const WenoFields W9) {
   if (!P.active(i, j, 1)) return;
   const cs_p1_patch& a = P.a;
   int64_t z6[6];
@@ -450,18 +464,17 @@ __global__ void __launch_bounds__(128) k_weno9(const P1 P, const Box b, const in
   }
 }
 
+// thread t: fields 3 (t / n) .. 3 (t / n) + 2 of zone t % n of the box
+__global__ void __launch_bounds__(128) k_weno9(const P1 P, const Box b, const WenoFields W9) {
+  const int64_t t = tid(), n = b.count();
+  if (t >= (int64_t)(W9.n / 3) * n) return;  // 3 or 9 fields
+  int i, j, k;
+  b.decode(t % n, i, j, k);
+  weno_group(P, i, j, k, P.zi(i, j, k), 3 * (int)(t / n), W9);
+}
+
 // ---------------------------------------------------------------------------
 // step 7.b: ENFORCE_PRESSURE_POSITIVITY_PRIM (440...f:6-830).
-// pass 0: every zone of the range with the incoming entropy means; sets fa and
-// counts the zones whose slopes were removed.
-// pass 1: the zones of a list (those with an fa zone earlier in the loop order
-// among their 27), taking the entropy means of the prev-flagged earlier zones
-// as zero; writes next and counts the zones whose flag changed.
-struct Flags {
-  uint8_t *fa, *prev, *next;
-  unsigned int* counter;
-};
-
 // the 27 zones around (i, j, k): the column and its 8 stencil neighbours
 // (R, L, U, D, RU, LU, LD, RD), each at k-1, k, k+1, as the zone index of
 // layer 0 of each column
@@ -482,19 +495,8 @@ __device__ __forceinline__ void columns9(const P1& P, int i, int j, int64_t* col
 // SIMD: at NM = 10 the registers are held to 256 with a small spill, which
 // the second wave more than pays for (the NM = 4 form fits without one)
 template <int NM>
-__global__ void __attribute__((amdgpu_waves_per_eu(2))) __launch_bounds__(256)
-    k_pos(const P1 P, const Box b, const int64_t* list, int64_t nlist, const Flags F, const double* __restrict__ mom) {
-  const int64_t t = tid();
-  int i, j, k;
-  int64_t z;
-  if (list) {
-    if (t >= nlist) return;
-    z = list[t];
-    zone_of(P, z, i, j, k);
-  } else {
-    if (!b.decode(t, i, j, k)) return;
-    z = P.zi(i, j, k);
-  }
+__device__ __forceinline__ void pos_zone(const P1& P, int i, int j, int k, int64_t z, int sweep, const Flags& F,
+                                         const double* __restrict__ mom) {
   const cs_p1_patch& a = P.a;
   int64_t col[9];
   columns9(P, i, j, col);
@@ -509,7 +511,7 @@ __global__ void __attribute__((amdgpu_waves_per_eu(2))) __launch_bounds__(256)
       const int64_t zz = col[q] + ks * (k + dk);
       const double r = P.V(0, 0, zz), p = P.V(4, 0, zz);
       double e = a.ent[zz];
-      if (list && zz < z && F.prev[zz]) e = 0.0;
+      if (sweep >= 0 && zz < z && F.fl[sweep & 1][zz]) e = 0.0;
       rmin = fmin(rmin, r);
       rmax = fmax(rmax, r);
       pmin = fmin(pmin, p);
@@ -671,49 +673,99 @@ __global__ void __attribute__((amdgpu_waves_per_eu(2))) __launch_bounds__(256)
     a.B3_zc[z + P.NZ * m] = P.V(7, m, z);
   }
   const uint8_t flag = removed ? 1 : 0;
-  if (!list) {
-    F.fa[z] = flag;
-    if (removed) atomicAdd(F.counter, 1u);
+  if (sweep < 0) {
+    F.fl[0][z] = flag;
+    F.fl[1][z] = flag;
+    F.ever[z] = flag;
+    if (removed) atomicAdd(&F.ctr[0], 1u);
   } else {
-    F.next[z] = flag;
-    if (flag != F.prev[z]) atomicAdd(F.counter, 1u);
+    F.fl[(sweep + 1) & 1][z] = flag;
+    if (flag) F.ever[z] = 1;
+    if (flag != F.fl[sweep & 1][z]) atomicAdd(&F.ctr[4 + sweep], 1u);
   }
+}
+template <int NM>
+__global__ void __attribute__((amdgpu_waves_per_eu(2))) __launch_bounds__(256)
+    k_pos(const P1 P, const Box b, const Flags F, const double* __restrict__ mom) {
+  int i, j, k;
+  if (!b.decode(tid(), i, j, k)) return;
+  pos_zone<NM>(P, i, j, k, P.zi(i, j, k), -1, F, mom);
 }
 
 // the zones of the range with a zone ever flagged earlier in the loop order
 // among their 27 and not yet on the list: appended to it (order immaterial;
 // the list only grows, so a zone whose result depends on a flag is
-// recomputed in every later sweep)
-__global__ void __launch_bounds__(256) k_cands(const P1 P, const Box b, const uint8_t* ever, uint8_t* inlist,
-                                               int64_t* list, unsigned int* count) {
-  int i, j, k;
-  if (!b.decode(tid(), i, j, k)) return;
-  const int64_t z = P.zi(i, j, k), ks = (int64_t)P.nz * P.nz;
-  if (inlist[z]) return;
-  int64_t col[9];
-  columns9(P, i, j, col);
-  bool cand = false;
-  for (int q = 0; q < 9; ++q)
+// recomputed in every later sweep; a zone that joins has its first pass's
+// flag in both arrays)
+constexpr int kListBlocks = 512;  // grids of the replay kernels (grid-stride)
+__global__ void __launch_bounds__(256) k_cands(const P1 P, const Box b, const Flags F, int sweep) {
+  if (F.done(sweep)) return;
+  const int64_t n = b.count(), ks = (int64_t)P.nz * P.nz;
+  for (int64_t t = tid(); t < n; t += (int64_t)gridDim.x * blockDim.x) {
+    int i, j, k;
+    b.decode(t, i, j, k);
+    const int64_t z = P.zi(i, j, k);
+    if (F.inlist[z]) continue;
+    int64_t col[9];
+    columns9(P, i, j, col);
+    bool cand = false;
+    for (int q = 0; q < 9; ++q)
 #pragma unroll
-    for (int dk = -1; dk <= 1; ++dk) {
-      const int64_t zz = col[q] + ks * (k + dk);
-      cand = cand || (zz < z && ever[zz]);
+      for (int dk = -1; dk <= 1; ++dk) {
+        const int64_t zz = col[q] + ks * (k + dk);
+        cand = cand || (zz < z && F.ever[zz]);
+      }
+    if (cand) {
+      F.inlist[z] = 1;
+      F.list[atomicAdd(&F.ctr[1], 1u)] = z;
     }
-  if (cand) {
-    inlist[z] = 1;
-    list[atomicAdd(count, 1u)] = z;
   }
 }
-
-// after a sweep: the list's new flags become the previous ones and join the
-// ever-flagged set
-__global__ void __launch_bounds__(256) k_commit(const int64_t* list, int64_t n, const uint8_t* next, uint8_t* prev,
-                                                uint8_t* ever) {
-  const int64_t t = tid();
-  if (t >= n) return;
-  const int64_t z = list[t];
-  prev[z] = next[z];
-  ever[z] = ever[z] | next[z];
+// one sweep over the list in groups of 64 zones: three waves redo their WENO
+// (three fields each), then the first wave their positivity.  The counts and
+// the flags stay on the device, so the host looks once per kSweepBatch sweeps
+// instead of twice per sweep (the call on a noisy 16^2 x 6 patch 423 -> 370 us,
+// 128^2 x 48 2.42 -> 2.29 ms)
+constexpr int kReplayZones = 64;
+__global__ void __attribute__((amdgpu_waves_per_eu(2))) __launch_bounds__(3 * kReplayZones)
+    k_replay(const P1 P, const Flags F, const WenoFields W9, int sweep) {
+  if (F.done(sweep)) return;
+  const int64_t n = F.ctr[1];
+  const int q = threadIdx.x % kReplayZones, grp = threadIdx.x / kReplayZones;
+  for (int64_t t0 = (int64_t)blockIdx.x * kReplayZones; t0 < n; t0 += (int64_t)gridDim.x * kReplayZones) {
+    const bool on = t0 + q < n;
+    int i = 0, j = 0, k = 0;
+    int64_t z = 0;
+    if (on) {
+      z = F.list[t0 + q];
+      zone_of(P, z, i, j, k);
+      weno_group(P, i, j, k, z, 3 * grp, W9);
+    }
+    __syncthreads();  // the zone's slopes are written before its positivity reads them
+    if (on && grp == 0) pos_zone<4>(P, i, j, k, z, sweep, F, nullptr);
+  }
+}
+// the same at third order in three launches, the WENO-AO (k_weno_ao_list) between
+__global__ void __launch_bounds__(128) k_weno9_list(const P1 P, const Flags F, const WenoFields W9, int sweep) {
+  if (F.done(sweep)) return;
+  const int64_t n = F.ctr[1];
+  for (int64_t t = tid(); t < 3 * n; t += (int64_t)gridDim.x * blockDim.x) {
+    const int64_t z = F.list[t % n];
+    int i, j, k;
+    zone_of(P, z, i, j, k);
+    weno_group(P, i, j, k, z, 3 * (int)(t / n), W9);
+  }
+}
+__global__ void __attribute__((amdgpu_waves_per_eu(2))) __launch_bounds__(256)
+    k_pos10_list(const P1 P, const Flags F, const double* __restrict__ mom, int sweep) {
+  if (F.done(sweep)) return;
+  const int64_t n = F.ctr[1];
+  for (int64_t t = tid(); t < n; t += (int64_t)gridDim.x * blockDim.x) {
+    const int64_t z = F.list[t];
+    int i, j, k;
+    zone_of(P, z, i, j, k);
+    pos_zone<10>(P, i, j, k, z, sweep, F, mom);
+  }
 }
 
 // the entropy means of the zones that lost all their slopes
@@ -1177,7 +1229,9 @@ __global__ void __launch_bounds__(kAoLanes * kAoGroups + 64)
     k_ao_e_sweep(const P1 P, const Box b, double* rec, double* xnew, unsigned int* ticket, int s);
 __global__ void __launch_bounds__(256) k_ao_e_put(const P1 P, const Box b, const double* __restrict__ rec);
 __global__ void __attribute__((amdgpu_waves_per_eu(2))) __launch_bounds__(128)
-    k_weno_ao(const P1 P, const Box b, const double* __restrict__ mom, const int64_t* list, int64_t nlist);
+    k_weno_ao(const P1 P, const Box b, const double* __restrict__ mom);
+__global__ void __attribute__((amdgpu_waves_per_eu(2))) __launch_bounds__(128)
+    k_weno_ao_list(const P1 P, const Box b, const double* __restrict__ mom, const Flags F, int sweep);
 }  // namespace csp1
 
 // mom (optional, DEVICE zone x 10): the third-order form, LIMIT_ALL_SLOPES_P12:
@@ -1216,7 +1270,8 @@ static int run_p1(const cs_p1_patch* p, void* stream_, float* kernel_ms, uint8_t
   const size_t flag_bytes = ((size_t)P.NZ + 255) / 256 * 256;
   const size_t list_bytes = (size_t)wr.count() * sizeof(int64_t);
   const Box ao = make_box(-1, N + 2, -1, N + 2, -1, NR + 2);
-  const size_t base_bytes = (5 * flag_bytes + 256 + (size_t)nblk_diag * 18 * sizeof(double) + 18 * sizeof(double) +
+  const size_t ctr_bytes = (kCtrWords * sizeof(unsigned int) + 255) / 256 * 256;
+  const size_t base_bytes = (4 * flag_bytes + ctr_bytes + (size_t)nblk_diag * 18 * sizeof(double) + 18 * sizeof(double) +
                              list_bytes + 255) / 256 * 256;
   const size_t need = base_bytes + (mom ? (size_t)ao.count() * (kAoRec + 4) * sizeof(double) : 0);
   if (mom && P.NZ >= ((int64_t)1 << 31)) {
@@ -1243,16 +1298,14 @@ static int run_p1(const cs_p1_patch* p, void* stream_, float* kernel_ms, uint8_t
     base = (uint8_t*)S.mem;
   }
   Flags F;
-  F.fa = base;
-  F.prev = base + flag_bytes;
-  F.next = base + 2 * flag_bytes;
-  uint8_t* ever = base + 3 * flag_bytes;    // flagged in the first pass or any sweep
-  uint8_t* inlist = base + 4 * flag_bytes;  // on the replay list
-  F.counter = (unsigned int*)(base + 5 * flag_bytes);
-  double* part = (double*)(base + 5 * flag_bytes + 256);
+  F.fl[0] = base;
+  F.fl[1] = base + flag_bytes;
+  F.ever = base + 2 * flag_bytes;
+  F.inlist = base + 3 * flag_bytes;
+  F.ctr = (unsigned int*)(base + 4 * flag_bytes);
+  double* part = (double*)(base + 4 * flag_bytes + ctr_bytes);
   double* red = part + (size_t)nblk_diag * 18;
-  int64_t* list = (int64_t*)(red + 18);
-  unsigned int* lcount = F.counter + 1;
+  F.list = (int64_t*)(red + 18);
   double* aorec = (double*)(base + base_bytes);  // third order: the records of k_ao_e_pre
 
   constexpr int NEV = CS_P1_STAGES + 1;
@@ -1267,7 +1320,7 @@ static int run_p1(const cs_p1_patch* p, void* stream_, float* kernel_ms, uint8_t
   };
   if ((rc = mark())) return rc;
   if (mom) k_zero_hi<<<grid_of(all.count(), 256), 256, 0, st>>>(P, all);
-  k_prim<<<grid_of(all.count(), 256), 256, 0, st>>>(P, all);
+  k_prim<<<grid_of(all.count(), 256), 256, 0, st>>>(P, all, F);
   if ((rc = mark())) return rc;
   k_face_zero<<<dim3(grid_of(P.NFC, 256), 3), 256, 0, st>>>(P);
   k_tricorner<<<grid_of(4 * (int64_t)g * P.nzr, 256), 256, 0, st>>>(P);
@@ -1276,9 +1329,6 @@ static int run_p1(const cs_p1_patch* p, void* stream_, float* kernel_ms, uint8_t
   k_flat_b<<<grid_of(all.count(), 256), 256, 0, st>>>(P, all);
   k_flat_c<<<grid_of(all.count(), 256), 256, 0, st>>>(P, all);
   if ((rc = mark())) return rc;
-  // flags of zones outside the limiter's range stay clear
-  P1_HIP(hipMemsetAsync(F.fa, 0, P.NZ, st));
-  P1_HIP(hipMemsetAsync(F.counter, 0, 2 * sizeof(unsigned int), st));
   WenoFields wv, we;
   wv.n = 9;
   wv.noflat = mom ? 0xffu : 0u;  // third order: V flattened after the hybridisation
@@ -1298,56 +1348,43 @@ static int run_p1(const cs_p1_patch* p, void* stream_, float* kernel_ms, uint8_t
     we.dst[c] = E3[c] + P.NZ;
     we.stride[c] = P.NZ;
   }
-  k_weno9<<<grid_of(3 * wr.count(), 128), 128, 0, st>>>(P, wr, nullptr, 0, wv);
+  k_weno9<<<grid_of(3 * wr.count(), 128), 128, 0, st>>>(P, wr, wv);
   if (mom) {
-    k_weno_ao<<<grid_of(ao.count(), 128), 128, 0, st>>>(P, ao, mom, nullptr, 0);
-    k_pos<10><<<grid_of(wr.count(), 256), 256, 0, st>>>(P, wr, nullptr, 0, F, mom);
+    k_weno_ao<<<grid_of(ao.count(), 128), 128, 0, st>>>(P, ao, mom);
+    k_pos<10><<<grid_of(wr.count(), 256), 256, 0, st>>>(P, wr, F, mom);
   } else {
-    k_pos<4><<<grid_of(wr.count(), 256), 256, 0, st>>>(P, wr, nullptr, 0, F, nullptr);
+    k_pos<4><<<grid_of(wr.count(), 256), 256, 0, st>>>(P, wr, F, nullptr);
   }
   P1_HIP(hipGetLastError());
   unsigned int nfail = 0;
-  P1_HIP(hipMemcpyAsync(&nfail, F.counter, sizeof(unsigned int), hipMemcpyDeviceToHost, st));
+  P1_HIP(hipMemcpyAsync(&nfail, F.ctr, sizeof(unsigned int), hipMemcpyDeviceToHost, st));
   P1_HIP(hipStreamSynchronize(st));
   if (nfail > 0) {
     // replay the loop-order dependence on the zones it can reach until the
     // flags settle: every sweep recomputes the list with the previous sweep's
     // flags; a zone newly flagged in a sweep brings its later neighbours
     // onto the list before the next one
-    P1_HIP(hipMemcpyAsync(F.prev, F.fa, P.NZ, hipMemcpyDeviceToDevice, st));
-    P1_HIP(hipMemcpyAsync(F.next, F.fa, P.NZ, hipMemcpyDeviceToDevice, st));
-    P1_HIP(hipMemcpyAsync(ever, F.fa, P.NZ, hipMemcpyDeviceToDevice, st));
-    P1_HIP(hipMemsetAsync(inlist, 0, P.NZ, st));
-    unsigned int ncand = 0;
-    bool settled = false;
-    for (int it = 0; it < 256 && !settled; ++it) {
-      k_cands<<<grid_of(wr.count(), 256), 256, 0, st>>>(P, wr, ever, inlist, list, lcount);
-      P1_HIP(hipMemsetAsync(F.counter, 0, sizeof(unsigned int), st));
-      P1_HIP(hipMemcpyAsync(&ncand, lcount, sizeof(unsigned int), hipMemcpyDeviceToHost, st));
-      P1_HIP(hipStreamSynchronize(st));
-      if (ncand == 0) {
-        settled = true;
-        break;
+    unsigned int nchg = 1;
+    for (int sw = 0; sw < kMaxSweeps && nchg > 0;) {
+      for (int q = 0; q < kSweepBatch; ++q, ++sw) {
+        k_cands<<<kListBlocks, 256, 0, st>>>(P, wr, F, sw);
+        if (mom) {
+          k_weno9_list<<<kListBlocks, 128, 0, st>>>(P, F, wv, sw);
+          k_weno_ao_list<<<kListBlocks, 128, 0, st>>>(P, ao, mom, F, sw);
+          k_pos10_list<<<kListBlocks, 256, 0, st>>>(P, F, mom, sw);
+        } else {
+          k_replay<<<kListBlocks, 3 * kReplayZones, 0, st>>>(P, F, wv, sw);
+        }
       }
-      k_weno9<<<grid_of(3 * (int64_t)ncand, 128), 128, 0, st>>>(P, wr, list, ncand, wv);
-      if (mom) {
-        k_weno_ao<<<grid_of(ncand, 128), 128, 0, st>>>(P, ao, mom, list, ncand);
-        k_pos<10><<<grid_of(ncand, 256), 256, 0, st>>>(P, wr, list, ncand, F, mom);
-      } else {
-        k_pos<4><<<grid_of(ncand, 256), 256, 0, st>>>(P, wr, list, ncand, F, nullptr);
-      }
-      k_commit<<<grid_of(ncand, 256), 256, 0, st>>>(list, ncand, F.next, F.prev, ever);
       P1_HIP(hipGetLastError());
-      unsigned int nchg = 0;
-      P1_HIP(hipMemcpyAsync(&nchg, F.counter, sizeof(unsigned int), hipMemcpyDeviceToHost, st));
+      P1_HIP(hipMemcpyAsync(&nchg, F.ctr + 4 + sw - 1, sizeof(unsigned int), hipMemcpyDeviceToHost, st));
       P1_HIP(hipStreamSynchronize(st));
-      settled = nchg == 0;
     }
-    if (!settled) {
+    if (nchg > 0) {
       cs::set_error("cs_limit_all_slopes_p1: positivity replay did not settle");
       return CS_E_INVALID;
     }
-    k_clear_ent<<<grid_of(wr.count(), 256), 256, 0, st>>>(P, wr, F.prev);
+    k_clear_ent<<<grid_of(wr.count(), 256), 256, 0, st>>>(P, wr, F.fl[0]);
   }
   if ((rc = mark())) return rc;
   if (mom)
@@ -1364,22 +1401,22 @@ static int run_p1(const cs_p1_patch* p, void* stream_, float* kernel_ms, uint8_t
     k_clsq_e<<<grid_of(all.count(), 64), 64, 0, st>>>(P, all);
   }
   if ((rc = mark())) return rc;
-  k_weno9<<<grid_of(wr.count(), 128), 128, 0, st>>>(P, wr, nullptr, 0, we);
+  k_weno9<<<grid_of(wr.count(), 128), 128, 0, st>>>(P, wr, we);
   if (mom) {
     // 9.c in the loop order of the reference's serial build (k_ao_e_sweep);
     // k_ao_order flags a stencil table for which a zone's earlier neighbours
     // are not all on lower levels and its later ones all on higher levels
+    // (F.ctr[2] and the sweep's ticket F.ctr[3] are clear since k_prim)
     double* xnew = aorec + (size_t)ao.count() * kAoRec;
     const int sj = ao_stride(ao.ni), threads = ((ao.ni + sj - 1) / sj * kAoLanes + 63) / 64 * 64 + 64;
-    P1_HIP(hipMemsetAsync(F.counter + 2, 0, 2 * sizeof(unsigned int), st));
-    k_ao_order<<<grid_of((int64_t)ao.ni * ao.nj, 256), 256, 0, st>>>(P, ao, F.counter + 2);
+    k_ao_order<<<grid_of((int64_t)ao.ni * ao.nj, 256), 256, 0, st>>>(P, ao, F.ctr + 2);
     k_ao_e_pre<<<grid_of(ao.count(), 128), 128, 0, st>>>(P, ao, mom, aorec, xnew);
-    k_ao_e_sweep<<<ao.nk, threads, 0, st>>>(P, ao, aorec, xnew, F.counter + 3, sj);
+    k_ao_e_sweep<<<ao.nk, threads, 0, st>>>(P, ao, aorec, xnew, F.ctr + 3, sj);
     k_ao_e_put<<<grid_of(ao.count(), 256), 256, 0, st>>>(P, ao, aorec);
   }
   if ((rc = mark())) return rc;
   k_diag<<<nblk_diag, DIAG_THREADS, 0, st>>>(P, all, part);
-  k_diag_final<<<18, 256, 0, st>>>(part, nblk_diag, red);
+  if (p->V_min_local || p->V_max_local) k_diag_final<<<18, 256, 0, st>>>(part, nblk_diag, red);
   if ((rc = mark())) return rc;
   P1_HIP(hipGetLastError());
   if (kernel_ms) {
@@ -1389,7 +1426,7 @@ static int run_p1(const cs_p1_patch* p, void* stream_, float* kernel_ms, uint8_t
   }
   if (mom) {
     unsigned int bad = 0;
-    P1_HIP(hipMemcpyAsync(&bad, F.counter + 2, sizeof(unsigned int), hipMemcpyDeviceToHost, st));
+    P1_HIP(hipMemcpyAsync(&bad, F.ctr + 2, sizeof(unsigned int), hipMemcpyDeviceToHost, st));
     P1_HIP(hipStreamSynchronize(st));
     if (bad) {
       cs::set_error("cs_limit_all_slopes_p12: the stencil table breaks the level order of step 9.c (an entry "
@@ -2843,17 +2880,7 @@ __device__ __forceinline__ constexpr int lt(int r, int c) { return r * (r + 1) /
 // (1 - flattener).  The reference inverts A^T A by LU (MATINV); the two
 // agree to rounding.  Two waves per SIMD, the registers held to 256 with a
 // small spill.
-__global__ void __attribute__((amdgpu_waves_per_eu(2))) __launch_bounds__(128)
-    k_weno_ao(const P1 P, const Box b, const double* __restrict__ mom, const int64_t* list, int64_t nlist) {
-  int i, j, k;
-  if (list) {  // the positivity replay's zones: those inside the range
-    const int64_t t = tid();
-    if (t >= nlist) return;
-    zone_of(P, list[t], i, j, k);
-    if (i < b.i0 || i >= b.i0 + b.ni || j < b.j0 || j >= b.j0 + b.nj || k < b.k0 || k >= b.k0 + b.nk) return;
-  } else if (!b.decode(tid(), i, j, k)) {
-    return;
-  }
+__device__ __forceinline__ void weno_ao_zone(const P1& P, int i, int j, int k, const double* __restrict__ mom) {
   if (!P.active(i, j, 1)) return;
   const cs_p1_patch& a = P.a;
   const int64_t z = P.zi(i, j, k), NZ = P.NZ;
@@ -2990,6 +3017,24 @@ __global__ void __attribute__((amdgpu_waves_per_eu(2))) __launch_bounds__(128)
 #pragma unroll
       for (int m = 3; m < 9; ++m) P.Vr(comp, m + 1, z) = whi * Phi[m] * x1;
     }
+  }
+}
+
+__global__ void __attribute__((amdgpu_waves_per_eu(2))) __launch_bounds__(128)
+    k_weno_ao(const P1 P, const Box b, const double* __restrict__ mom) {
+  int i, j, k;
+  if (b.decode(tid(), i, j, k)) weno_ao_zone(P, i, j, k, mom);
+}
+// the positivity replay's zones inside the range
+__global__ void __attribute__((amdgpu_waves_per_eu(2))) __launch_bounds__(128)
+    k_weno_ao_list(const P1 P, const Box b, const double* __restrict__ mom, const Flags F, int sweep) {
+  if (F.done(sweep)) return;
+  const int64_t n = F.ctr[1];
+  for (int64_t t = tid(); t < n; t += (int64_t)gridDim.x * blockDim.x) {
+    int i, j, k;
+    zone_of(P, F.list[t], i, j, k);
+    if (i < b.i0 || i >= b.i0 + b.ni || j < b.j0 || j >= b.j0 + b.nj || k < b.k0 || k >= b.k0 + b.nk) continue;
+    weno_ao_zone(P, i, j, k, mom);
   }
 }
 
