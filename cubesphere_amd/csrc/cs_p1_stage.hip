@@ -234,7 +234,9 @@ __global__ void __launch_bounds__(256) k_prim(Dev D, Box b, Buf6 in) {
   const int s = wg.y;
   const int64_t z = D.zi(i, j, k);
   const bool act = D.active(i, j);
-  double U[8], Vv[8];
+  double U[8], was[8], Vv[8];
+#pragma unroll
+  for (int c = 0; c < 8; ++c) was[c] = in.u(D, s, c, z);
   if (!act) {
 #pragma unroll
     for (int c = 0; c < 8; ++c) U[c] = 0.0;
@@ -242,7 +244,7 @@ __global__ void __launch_bounds__(256) k_prim(Dev D, Box b, Buf6 in) {
     U[4] = D.prsfloor / (D.gamma - 1.0);
   } else {
 #pragma unroll
-    for (int c = 0; c < 8; ++c) U[c] = in.u(D, s, c, z);
+    for (int c = 0; c < 8; ++c) U[c] = was[c];
   }
   double e = in.e(D, s, z);
   const Gas<double> gs = D.gas();
@@ -250,7 +252,7 @@ __global__ void __launch_bounds__(256) k_prim(Dev D, Box b, Buf6 in) {
   cons_to_prim(gs, U, Vv, e);
 #pragma unroll
   for (int c = 0; c < 8; ++c) {
-    in.u(D, s, c, z) = U[c];
+    put_changed(in.u(D, s, c, z), U[c], was[c]);
     D.v(0, s, c, z) = Vv[c];
   }
   in.e(D, s, z) = e;

@@ -156,7 +156,9 @@ __global__ void __launch_bounds__(256) k_prim(const P1 P, const Box b, const Fla
     }
 #pragma unroll
   for (int m = 1; m < 4; ++m) a.ent[z + P.NZ * m] = 0.0;
-  double U[8], V[8];
+  double U[8], was[8], V[8];
+#pragma unroll
+  for (int c = 0; c < 8; ++c) was[c] = P.Ur(c, 0, z);
   if (a.mask[z] == 0) {
 #pragma unroll
     for (int c = 0; c < 8; ++c) U[c] = 0.0;
@@ -165,7 +167,7 @@ __global__ void __launch_bounds__(256) k_prim(const P1 P, const Box b, const Fla
     a.scale[z] = a.smallnum;
   } else {
 #pragma unroll
-    for (int c = 0; c < 8; ++c) U[c] = P.Ur(c, 0, z);
+    for (int c = 0; c < 8; ++c) U[c] = was[c];
   }
   double e = a.ent[z];
   Gas<double> gs{gam, gam - 1.0, a.rhofloor, a.prsfloor, 1.0 / (gam - 1.0)};
@@ -174,7 +176,7 @@ __global__ void __launch_bounds__(256) k_prim(const P1 P, const Box b, const Fla
 #pragma unroll
   for (int c = 0; c < 8; ++c) {
     P.Vr(c, 0, z) = V[c];
-    P.Ur(c, 0, z) = U[c];
+    put_changed(P.Ur(c, 0, z), U[c], was[c]);
   }
   a.ent[z] = e;
   const double b2 = (V[5] * V[5] + V[6] * V[6] + V[7] * V[7]) * C<double>::ob4pi;
@@ -2143,7 +2145,9 @@ __global__ void __launch_bounds__(256) k_cleanup_zone(const P1 P) {
     }
 #pragma unroll
   for (int m = 1; m < 4; ++m) a.ent[z + P.NZ * m] = 0.0;
-  double U[8], V[8];
+  double U[8], was[8], V[8];
+#pragma unroll
+  for (int c = 0; c < 8; ++c) was[c] = P.Ur(c, 0, z);
   if (a.mask[z] == 0) {
 #pragma unroll
     for (int c = 0; c < 8; ++c) U[c] = 0.0;
@@ -2152,7 +2156,7 @@ __global__ void __launch_bounds__(256) k_cleanup_zone(const P1 P) {
     a.scale[z] = a.smallnum;
   } else {
 #pragma unroll
-    for (int c = 0; c < 8; ++c) U[c] = P.Ur(c, 0, z);
+    for (int c = 0; c < 8; ++c) U[c] = was[c];
   }
   if (P.active(i, j, 1)) {
     // rows: x+ and x- face normals, y+ and y-, and the radial direction of
@@ -2220,7 +2224,7 @@ __global__ void __launch_bounds__(256) k_cleanup_zone(const P1 P) {
 #pragma unroll
   for (int c = 0; c < 8; ++c) {
     P.Vr(c, 0, z) = V[c];
-    P.Ur(c, 0, z) = U[c];
+    put_changed(P.Ur(c, 0, z), U[c], was[c]);
   }
   a.ent[z] = e;
 }
@@ -2252,15 +2256,15 @@ __global__ void __launch_bounds__(DT_THREADS) k_dt(const P1 P, const Box own, do
     own.decode(t, i, j, k);
     const int64_t z = P.zi(i, j, k);
     if (a.mask[z] == 0) continue;
-    double U[8], V[8];
+    double U[8], was[8], V[8];
 #pragma unroll
-    for (int c = 0; c < 8; ++c) U[c] = P.Ur(c, 0, z);
+    for (int c = 0; c < 8; ++c) U[c] = was[c] = P.Ur(c, 0, z);
     double e = a.ent[z];  // the routine keeps its entropy array as it is
     V[4] = 0.0;
     cons_to_prim(gs, U, V, e);
 #pragma unroll
     for (int c = 0; c < 8; ++c) {
-      P.Ur(c, 0, z) = U[c];
+      put_changed(P.Ur(c, 0, z), U[c], was[c]);
       P.Vr(c, 0, z) = V[c];
     }
     const double b2 = V[5] * V[5] + V[6] * V[6] + V[7] * V[7];
