@@ -39,6 +39,7 @@
 
 #include <algorithm>
 #include <mutex>
+#include <type_traits>
 #include <vector>
 
 #include "cs_physics.h"
@@ -1128,7 +1129,9 @@ static inline unsigned grid_of(int64_t n, int threads) { return (unsigned)((n + 
 // instead of the library's per-device allocation (no allocation then)
 namespace csp1 {
 __global__ void __launch_bounds__(256) k_zero_hi(const P1 P, const Box b);
-__global__ void __launch_bounds__(64) k_clsq12(const P1 P, const Box b, const double* __restrict__ mom);
+__global__ void __attribute__((amdgpu_waves_per_eu(2))) __launch_bounds__(64)
+    k_clsq12(const P1 P, const Box b, const double* __restrict__ mom);
+constexpr int kSqZones = 4;  // zones per wave of k_clsq12
 __global__ void __launch_bounds__(256) k_e12(const P1 P, const Box b, const double* __restrict__ mom);
 __global__ void __launch_bounds__(256) k_ao_order(const P1 P, const Box b, unsigned int* bad);
 constexpr int kAoRec = 208;     // doubles per zone record of k_ao_e_pre
@@ -1312,7 +1315,7 @@ static int run_p1(const cs_p1_patch* p, void* stream_, float* kernel_ms, uint8_t
         P, fx, fy, fz, nullptr);
   if ((rc = mark())) return rc;
   if (mom) {
-    k_clsq12<<<(unsigned)wr.count(), 64, 0, st>>>(P, wr, mom);
+    k_clsq12<<<grid_of(wr.count(), kSqZones), 64, 0, st>>>(P, wr, mom);
     k_e12<<<grid_of(all.count(), 256), 256, 0, st>>>(P, all, mom);
   } else {
     k_clsq_e<<<grid_of(all.count(), 64), 64, 0, st>>>(P, all);
@@ -2957,200 +2960,276 @@ __global__ void __attribute__((amdgpu_waves_per_eu(2))) __launch_bounds__(128)
   }
 }
 
-// Step 8.d at third order (421...f:5574-6680), one wave per zone: the 36 x 36
-// system of the normal equations of the 64 least-squares rows (n . B at the
-// 30 face points against their face-point B, the 30 WENO-AO modes, the
-// divergence and its gradient) and the 6 face-mean constraints.  Lanes 0-29
-// put one face point each (normal, the ten basis values about the zone's
-// moments, B-field weight, face-point B) in LDS; lane r < 36 forms row r of
-// the augmented system in registers (A^T A = P^T P + I + D^T D, P the point
-// rows, D the divergence rows; P^T P by FP64 MFMA across the wave); Gaussian
-// elimination across the lanes in natural order, then back substitution.  The
-// reference solves the same system by Numerical Recipes' LU with partial
-// pivoting (MATSOLVE): the two
-// agree to rounding.
-// lane l's value of v, uniform across the wave (l uniform)
-__device__ __forceinline__ double rdlane(double v, int l) {
-  const long long b = __double_as_longlong(v);
-  const unsigned int lo = (unsigned int)__builtin_amdgcn_readlane((int)(unsigned int)b, l);
-  const unsigned int hi = (unsigned int)__builtin_amdgcn_readlane((int)(b >> 32), l);
-  return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+// LDS words written before by a wave's lanes, read after by its others
+__device__ __forceinline__ void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-__constant__ double c_div_rows[4][30] = {
-    {0, 1, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 1, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 1, 0, 0, 0, 0, 0, 0},
-    {0, 0, 0, 0, 2, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 1, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 1},
-    {0, 0, 0, 0, 0, 0, 0, 1, 0, 0, 0, 0, 0, 0, 0, 2, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 1, 0},
-    {0, 0, 0, 0, 0, 0, 0, 0, 0, 1, 0, 0, 0, 0, 0, 0, 0, 0, 1, 0, 0, 0, 0, 0, 0, 0, 2, 0, 0, 0}};
+// Step 8.d at third order (421...f:5574-6680), four zones per wave, 16 lanes
+// each: the 36 x 36 system of the normal equations of the 64 least-squares
+// rows (n . B at the 30 face points against their face-point B, the 30 WENO-AO
+// modes, the divergence and its gradient) and the 6 face-mean constraints.
+// The face points' words (normal, the ten basis values about the zone's
+// moments, B-field weight, face-point B) go through LDS; lane r holds the rows
+// r, r + 16 and r + 32 of the lower triangle (K = P^T P + I + D^T D above the
+// constraint rows C) in registers, 84 doubles.  L D L^T in natural order: the
+// leading 30 x 30 block has every eigenvalue at least 1, so its pivots are too,
+// and the trailing block then holds -C K^-1 C^T, negative definite for the six
+// independent rows C, so no pivot search is needed.  A column entry reaches
+// the zone's lanes by a row broadcast (DPP), a row of L the back substitution
+// through LDS, where its words have taken the face points' place.  The
+// reference solves the same system by Numerical Recipes' LU with partial
+// pivoting (MATSOLVE): the two agree to rounding.
+//
+// One zone per wave with the whole rows in 36 lanes and v_readlane broadcasts
+// (the Gram by FP64 MFMA) spent two broadcast instructions on each multiply-add
+// and eliminated both triangles: 64^2 x 25 1.34 -> 0.60 ms, 192^2 x 64 22.5 ->
+// 10.5 ms with k_e12, 49,644 operations a zone at 13.0 TFLOP/s.  What bounds
+// it now is FP64 issue at two waves per SIMD (1,500 multiply-adds and as many
+// broadcast moves per four zones); the point loop unrolled five-fold spills
+// (0.69 ms at 64^2 x 25).  Against the system in 80-bit arithmetic its largest
+// relative error is 4.0e-15, the earlier form's 4.2e-15.
+constexpr int kSqStride = 484;    // LDS words per zone: 30 points of 16, and 4 against bank conflicts
 
-__global__ void __launch_bounds__(64) k_clsq12(const P1 P, const Box b, const double* __restrict__ mom) {
-  // one LDS block: the face points' words first (pt), then the Gram (gram),
-  // which is written after the last read of pt; 8.4 KB per zone instead of
-  // 12.3, so more zones fit a CU than its registers allow anyway
-  __shared__ double sh[32 * 33];
-  double(*pt)[16] = reinterpret_cast<double(*)[16]>(sh);  // n (3), basis (10), weight, face-point B
-  const int lane = threadIdx.x;
+// lane N of each row of 16 lanes, in all of them
+template <int N>
+__device__ __forceinline__ double row_lane(double v) {
+  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), 0x150 + N, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), 0x150 + N, 0xf, 0xf, true);
+  return __hiloint2double(hi, lo);
+}
+// f(integral_constant) for I = A .. B - 1
+template <int A, int B, class F>
+__device__ __forceinline__ void static_for(const F& f) {
+  if constexpr (A < B) {
+    f(std::integral_constant<int, A>{});
+    static_for<A + 1, B>(f);
+  }
+}
+
+__global__ void __attribute__((amdgpu_waves_per_eu(2))) __launch_bounds__(64)
+    k_clsq12(const P1 P, const Box b, const double* __restrict__ mom) {
+  __shared__ double2 sh[kSqZones * kSqStride / 2];
+  const int r = threadIdx.x % 16, g = threadIdx.x / 16;
   int i, j, k;
-  if (!b.decode(blockIdx.x, i, j, k)) return;  // one zone per workgroup: uniform
+  if (!b.decode((int64_t)blockIdx.x * kSqZones + g, i, j, k)) return;  // all 16 lanes of a zone
   const cs_p1_patch& a = P.a;
   const int64_t z = P.zi(i, j, k), NZ = P.NZ;
   if (a.mask[z] == 0) return;
-  const double obl = P.obl(z);
-  double c0[10];
-#pragma unroll
-  for (int m = 0; m < 10; ++m) c0[m] = mom[z + NZ * m];
-  if (lane < 30) {
-    const int f = lane / 5, q = lane % 5, fam = f >> 1;
-    const bool hi = (f & 1) == 0;
-    const int fi = i - (fam == 0 && !hi), fj = j - (fam == 1 && !hi), fk = k - (fam == 2 && !hi);
-    const int64_t fg = fam == 0 ? P.xfi(fi, fj, fk) : (fam == 1 ? P.yfi(fi, fj, fk) : P.zfi(fi, fj, fk));
-    const int64_t NF = fam == 2 ? P.NZF : P.NXF, fb = P.fci(fi, fj, fk);
-    const double* nrm = fam == 0 ? a.xb_normal : (fam == 1 ? a.yb_normal : a.zb_normal);
-    const double* pts = fam == 0 ? a.xb_pts : (fam == 1 ? a.yb_pts : a.zb_pts);
-    const double* wts = fam == 0 ? a.xb_wts : (fam == 1 ? a.yb_wts : a.zb_wts);
-    const double* Bq = fam == 0 ? a.Bxf_q : (fam == 1 ? a.Byf_q : a.Bzf_q);
-    double r[3];
-#pragma unroll
-    for (int c = 0; c < 3; ++c) {
-      pt[lane][c] = fam == 2 ? nrm[fg + NF * (c + 3 * q)] : nrm[fg + NF * c];
-      r[c] = (pts[fg + NF * (c + 3 * q)] - P.cen(z, c)) * obl;
-    }
-    pt[lane][3] = 1.0;
-    pt[lane][4] = r[0];
-    pt[lane][5] = r[1];
-    pt[lane][6] = r[2];
-    pt[lane][7] = r[0] * r[0] - c0[4];
-    pt[lane][8] = r[1] * r[1] - c0[5];
-    pt[lane][9] = r[2] * r[2] - c0[6];
-    pt[lane][10] = r[0] * r[1] - c0[7];
-    pt[lane][11] = r[1] * r[2] - c0[8];
-    pt[lane][12] = r[0] * r[2] - c0[9];
-    pt[lane][13] = wts[fg + NF * q];
-    pt[lane][14] = Bq[fb + P.NFC * q];
-  }
-  __syncthreads();
-  // row `lane` of the augmented system [K | rhs]
-  double row[37];
-#pragma unroll
-  for (int e = 0; e < 37; ++e) row[e] = 0.0;
-  if (lane < 30) {
-    const int c = lane / 10, m = lane % 10;
-#pragma unroll
-    for (int e = 0; e < 30; ++e) {
-      double t = e == lane ? 1.0 : 0.0;
-#pragma unroll
-      for (int d = 0; d < 4; ++d) t += c_div_rows[d][lane] * c_div_rows[d][e];
-      row[e] = t;
-    }
-    row[36] = P.V(5 + c, m, z);
-#pragma unroll
-    for (int f = 0; f < 6; ++f) {
-      double cf = 0.0;  // the constraint column of face f
-#pragma unroll
-      for (int q = 5 * f; q < 5 * f + 5; ++q) {
-        const double pa = pt[q][c] * pt[q][3 + m];
-        row[36] += pa * pt[q][14];
-        cf += pt[q][13] * pa;
-      }
-      row[30 + f] = cf;
-    }
-  } else if (lane < 36) {
-    const int f = lane - 30;
-#pragma unroll
-    for (int q5 = 0; q5 < 5; ++q5) {
-      const int q = 5 * f + q5;
-      const double w = pt[q][13];
-#pragma unroll
-      for (int cc = 0; cc < 3; ++cc) {
-        const double wn = w * pt[q][cc];
-#pragma unroll
-        for (int mm = 0; mm < 10; ++mm) row[10 * cc + mm] += wn * pt[q][3 + mm];
-      }
-      row[36] += w * pt[q][14];
-    }
-  }
-  // P^T P, the Gram of the 30 point rows P[q][10 c + m] = n_c(q) basis_m(q),
-  // by FP64 MFMA 16 x 16 x 4 over the zero-padded 32 x 32: lane l brings
-  // P[4 kc + l / 16][16 I + l % 16] as both operands (A = P^T by columns, B = P
-  // by rows), and result register r of lane l is entry (l / 16 + 4 r, l % 16)
-  // of its 16 x 16 block.  Blocks (0, 0), (0, 1) and (1, 1) are formed, (1, 0)
-  // is (0, 1) transposed; the sum goes through LDS to the row lanes.
-  double(*gram)[33] = reinterpret_cast<double(*)[33]>(sh);
+  double* const pt = (double*)sh + g * kSqStride;  // [30][16]: n (3), basis (10), weight, face-point B
   {
-    typedef double d4 __attribute__((ext_vector_type(4)));
-    d4 g00 = {0.0, 0.0, 0.0, 0.0}, g01 = g00, g11 = g00;
-    const int l16 = lane % 16, lq = lane / 16;
+    const double obl = P.obl(z);
+    double c0[6];
 #pragma unroll
-    for (int kc = 0; kc < 8; ++kc) {
-      const int q = 4 * kc + lq;
-      double p0 = 0.0, p1 = 0.0;
-      if (q < 30) {
-        p0 = pt[q][l16 / 10] * pt[q][3 + l16 % 10];
-        if (16 + l16 < 30) p1 = pt[q][(16 + l16) / 10] * pt[q][3 + (16 + l16) % 10];
+    for (int m = 0; m < 6; ++m) c0[m] = mom[z + NZ * (4 + m)];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int pq = r + 16 * h;
+      if (pq < 30) {
+        const int f = pq / 5, q = pq % 5, fam = f >> 1;
+        const bool hi = (f & 1) == 0;
+        const int fi = i - (fam == 0 && !hi), fj = j - (fam == 1 && !hi), fk = k - (fam == 2 && !hi);
+        const int64_t fg = fam == 0 ? P.xfi(fi, fj, fk) : (fam == 1 ? P.yfi(fi, fj, fk) : P.zfi(fi, fj, fk));
+        const int64_t NF = fam == 2 ? P.NZF : P.NXF, fb = P.fci(fi, fj, fk);
+        const double* nrm = fam == 0 ? a.xb_normal : (fam == 1 ? a.yb_normal : a.zb_normal);
+        const double* pts = fam == 0 ? a.xb_pts : (fam == 1 ? a.yb_pts : a.zb_pts);
+        const double* wts = fam == 0 ? a.xb_wts : (fam == 1 ? a.yb_wts : a.zb_wts);
+        const double* Bq = fam == 0 ? a.Bxf_q : (fam == 1 ? a.Byf_q : a.Bzf_q);
+        double x[3];
+        double* w = pt + 16 * pq;
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+          w[c] = fam == 2 ? nrm[fg + NF * (c + 3 * q)] : nrm[fg + NF * c];
+          x[c] = (pts[fg + NF * (c + 3 * q)] - P.cen(z, c)) * obl;
+        }
+        w[3] = 1.0;
+        w[4] = x[0];
+        w[5] = x[1];
+        w[6] = x[2];
+        w[7] = x[0] * x[0] - c0[0];
+        w[8] = x[1] * x[1] - c0[1];
+        w[9] = x[2] * x[2] - c0[2];
+        w[10] = x[0] * x[1] - c0[3];
+        w[11] = x[1] * x[2] - c0[4];
+        w[12] = x[0] * x[2] - c0[5];
+        w[13] = wts[fg + NF * q];
+        w[14] = Bq[fb + P.NFC * q];
       }
-      g00 = __builtin_amdgcn_mfma_f64_16x16x4f64(p0, p0, g00, 0, 0, 0);
-      g01 = __builtin_amdgcn_mfma_f64_16x16x4f64(p0, p1, g01, 0, 0, 0);
-      g11 = __builtin_amdgcn_mfma_f64_16x16x4f64(p1, p1, g11, 0, 0, 0);
-    }
-    __syncthreads();  // pt is read no more: the Gram takes its place
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int gr = lq + 4 * r;
-      gram[gr][l16] = g00[r];
-      gram[gr][16 + l16] = g01[r];
-      gram[16 + l16][gr] = g01[r];
-      gram[16 + gr][16 + l16] = g11[r];
     }
   }
-  __syncthreads();
-  if (lane < 30) {
+  wave_sync();
+  // rows r and r + 16 (r < 14) of K: their component and mode
+  const int ca = r / 10, ma = r % 10, cb = r < 14 ? (r + 16) / 10 : 0, mb = r < 14 ? (r + 16) % 10 : 0;
+  double K0[16], K1[32], K2[36], y0, y1, y2 = 0.0;
 #pragma unroll
-    for (int e = 0; e < 30; ++e) row[e] += gram[lane][e];
-  }
-  // Elimination in natural order, lane jj holding pivot row jj: the leading
-  // 30 x 30 block is I + D^T D + P^T P, symmetric positive definite with
-  // every eigenvalue at least 1, so its pivots are too; the trailing 6 x 6
-  // block then holds -C K^-1 C^T, negative definite for the six independent
-  // face-mean rows C.  No pivot search, and the pivot row comes from a known
-  // lane, broadcast through scalar registers.
+  for (int e = 0; e < 16; ++e) K0[e] = e == r ? 1.0 : 0.0;
 #pragma unroll
-  for (int jj = 0; jj < 36; ++jj) {
-    // the whole pivot row first, then the updates: the scalar registers the
-    // broadcasts write are read well after, without wait states between
-    double pr[37];
+  for (int e = 0; e < 32; ++e) K1[e] = e == r + 16 && r < 14 ? 1.0 : 0.0;
+  y0 = P.V(5 + ca, ma, z);
+  y1 = r < 14 ? P.V(5 + cb, mb, z) : 0.0;
+  // the Gram of the point rows, their right-hand side; a finished face's
+  // points make room for its constraint row
+#pragma unroll 1
+  for (int f = 0; f < 6; ++f) {
+    double Ca = 0.0, Cb = 0.0, d = 0.0;
+#pragma unroll 1
+    for (int q = 0; q < 5; ++q) {
+      const double* w = pt + 16 * (5 * f + q);
+      const double pa = w[ca] * w[3 + ma], pb = r < 14 ? w[cb] * w[3 + mb] : 0.0;
+      double v[16];
 #pragma unroll
-    for (int e = jj; e < 37; ++e) pr[e] = rdlane(row[e], jj);
-    const double fct = row[jj] / pr[jj];
-    if (lane > jj) {
+      for (int h = 0; h < 8; ++h) {
+        const double2 t = ((const double2*)w)[h];
+        v[2 * h] = t.x;
+        v[2 * h + 1] = t.y;
+      }
 #pragma unroll
-      for (int e = jj + 1; e < 37; ++e) row[e] -= fct * pr[e];
+      for (int c = 0; c < 3; ++c) {
+        const double na = pa * v[c], nb = pb * v[c];
+#pragma unroll
+        for (int m = 0; m < 10; ++m) {
+          if (10 * c + m < 16) K0[10 * c + m] += na * v[3 + m];
+          K1[10 * c + m] += nb * v[3 + m];
+        }
+      }
+      y0 += pa * v[14];
+      y1 += pb * v[14];
+      Ca += v[13] * pa;
+      Cb += v[13] * pb;
+      d += v[13] * v[14];
     }
+    wave_sync();
+    pt[80 * f + r] = Ca;
+    pt[80 * f + 16 + r] = Cb;
+    wave_sync();
+    if (r == 14 + f) y1 = d;  // f = 0, 1
+    if (r == f - 2) y2 = d;   // f = 2 .. 5
   }
-  // back substitution by columns: x[jj] from lane jj, then every lane above
-  // takes it out of its right-hand side
-  double x[36];
+  // the constraint rows: 30 and 31 in the second set, 32 to 35 in the third
 #pragma unroll
-  for (int jj = 35; jj >= 0; --jj) {
-    x[jj] = rdlane(row[36] / row[jj], jj);
-    if (lane < jj) row[36] -= row[jj] * x[jj];
+  for (int e = 0; e < 30; ++e) {
+    const double t1 = pt[80 * (r >= 14 ? r - 14 : 0) + e], t2 = pt[80 * (r < 4 ? r + 2 : 2) + e];
+    K1[e] = r >= 14 ? t1 : K1[e];
+    K2[e] = r < 4 ? t2 : 0.0;
   }
-  if (lane < 30) {
-    const int c = lane / 10, m = lane % 10;
+#pragma unroll
+  for (int e = 30; e < 36; ++e) K2[e] = 0.0;
+  // D^T D of the four divergence rows (421...f:6000-6200): row d has 1 at three
+  // modes, 2 at the own quadratic one
+  {
+    auto dv = [](int row, int e1, int e2, int e3, int two) {
+      return (row == e1 || row == e2 || row == e3) ? (row == two ? 2.0 : 1.0) : 0.0;
+    };
+    auto add = [&](int row, auto& K, auto limit) {
+      constexpr int n = decltype(limit)::value;
+      const double d0 = dv(row, 1, 12, 23, -1), d1 = dv(row, 4, 17, 29, 4), d2 = dv(row, 7, 15, 28, 15),
+                   d3 = dv(row, 9, 18, 26, 26);
+      K[1] += d0;
+      K[4] += 2.0 * d1;
+      K[7] += d2;
+      K[9] += d3;
+      K[12] += d0;
+      K[15] += 2.0 * d2;
+      if constexpr (n > 16) {
+        K[17] += d1;
+        K[18] += d3;
+        K[23] += d0;
+        K[26] += 2.0 * d3;
+        K[28] += d2;
+        K[29] += d1;
+      }
+    };
+    add(r, K0, std::integral_constant<int, 16>{});
+    add(r < 14 ? r + 16 : -1, K1, std::integral_constant<int, 32>{});
+  }
+  // elimination: step jj takes row jj out of the rows below it.  The entries
+  // of column jj are the multipliers times the pivot; a lane whose row is jj
+  // or above takes none
+  static_for<0, 36>([&](auto J) {
+    constexpr int jj = J, ps = jj / 16, pl = jj % 16;
+    double col[3] = {ps == 0 ? K0[ps == 0 ? jj : 0] : 0.0, ps <= 1 ? K1[ps <= 1 ? jj : 0] : 0.0, K2[jj]};
+    const double piv = row_lane<pl>(col[ps]), od = 1.0 / piv;
+    double mul[3];
+#pragma unroll
+    for (int s = 0; s < 3; ++s) mul[s] = s < ps ? 0.0 : col[s] * od;
+    if (r <= pl) mul[ps] = 0.0;
+    const double yj = row_lane<pl>(ps == 0 ? y0 : (ps == 1 ? y1 : y2));
+    if constexpr (ps == 0) y0 = r == pl ? y0 * od : y0 - mul[0] * yj;
+    if constexpr (ps == 1) y1 = r == pl ? y1 * od : y1 - mul[1] * yj;
+    if constexpr (ps == 2) y2 = r == pl ? y2 * od : y2 - mul[2] * yj;
+    if constexpr (ps < 1) y1 -= mul[1] * yj;
+    if constexpr (ps < 2) y2 -= mul[2] * yj;
+    static_for<jj + 1, 36>([&](auto E) {
+      constexpr int e = E;
+      const double v = row_lane<e % 16>(col[e / 16]);
+      if constexpr (e < 16) K0[e] -= mul[0] * v;
+      if constexpr (e < 32 && ps <= 1) K1[e] -= mul[1] * v;
+      K2[e] -= mul[2] * v;
+    });
+    if constexpr (ps == 0) K0[jj] = mul[0];
+    if constexpr (ps <= 1) K1[jj] = mul[1];
+    K2[jj] = mul[2];
+  });
+  // back substitution with the rows of L from LDS: the third set, then the
+  // second's own block, its part in the first's unknowns, the first
+  double* const lt = pt;
+  wave_sync();
+  if (r < 4) {
+#pragma unroll
+    for (int e = 0; e < 36; ++e) lt[37 * r + e] = K2[e];
+  }
+  wave_sync();
+  static_for<0, 4>([&](auto J) {
+    constexpr int q = 3 - J;
+    const double x = row_lane<q>(y2);
+    y0 -= lt[37 * q + r] * x;
+    y1 -= lt[37 * q + 16 + r] * x;
+    const double t = lt[37 * q + 32 + (r < 4 ? r : 0)];
+    if (r < q) y2 -= t * x;
+  });
+  wave_sync();
+#pragma unroll
+  for (int e = 0; e < 16; ++e) lt[17 * r + e] = K1[16 + e];
+  wave_sync();
+  static_for<0, 16>([&](auto J) {
+    constexpr int q = 15 - J;
+    const double x = row_lane<q>(y1), t = lt[17 * q + r];
+    if (r < q) y1 -= t * x;
+  });
+  wave_sync();
+#pragma unroll
+  for (int e = 0; e < 16; ++e) lt[17 * r + e] = K1[e];
+  wave_sync();
+  static_for<0, 16>([&](auto J) {
+    constexpr int q = J;
+    y0 -= lt[17 * q + r] * row_lane<q>(y1);
+  });
+  wave_sync();
+#pragma unroll
+  for (int e = 0; e < 16; ++e) lt[17 * r + e] = K0[e];
+  wave_sync();
+  static_for<0, 16>([&](auto J) {
+    constexpr int q = 15 - J;
+    const double x = row_lane<q>(y0), t = lt[17 * q + r];
+    if (r < q) y0 -= t * x;
+  });
+  auto out = [&](int c, int m, double v) {
     double* Bz = c == 0 ? a.B1_zc : (c == 1 ? a.B2_zc : a.B3_zc);
-    double mine = x[0];
-#pragma unroll
-    for (int e = 1; e < 30; ++e)
-      if (e == lane) mine = x[e];
-    Bz[z + NZ * m] = mine;
-    P.Vr(5 + c, m, z) = mine;
-  }
-  if (lane == 0) {
+    Bz[z + NZ * m] = v;
+    P.Vr(5 + c, m, z) = v;
+  };
+  out(ca, ma, y0);
+  if (r < 14) out(cb, mb, y1);
+  const double b0 = row_lane<0>(y0), b1 = row_lane<10>(y0), b2 = row_lane<4>(y1);
+  if (r == 0) {
     const double ob8pi = 1.0 / (8.0 * M_PI);
     const double aa = (P.Ur(5, 0, z) * P.Ur(5, 0, z) + P.Ur(6, 0, z) * P.Ur(6, 0, z) + P.Ur(7, 0, z) * P.Ur(7, 0, z)) * ob8pi;
-    P.Ur(5, 0, z) = x[0];
-    P.Ur(6, 0, z) = x[10];
-    P.Ur(7, 0, z) = x[20];
-    const double bb = (x[0] * x[0] + x[10] * x[10] + x[20] * x[20]) * ob8pi;
+    P.Ur(5, 0, z) = b0;
+    P.Ur(6, 0, z) = b1;
+    P.Ur(7, 0, z) = b2;
+    const double bb = (b0 * b0 + b1 * b1 + b2 * b2) * ob8pi;
     P.Ur(4, 0, z) = P.Ur(4, 0, z) - aa + bb;
   }
 }
@@ -3452,12 +3531,6 @@ __device__ __forceinline__ double row_sum(double v) {
   v = dpp_add<0x4e>(v);       // quad_perm 2 3 0 1
   v = dpp_add<0x141>(v);      // row_half_mirror
   return dpp_add<0x140>(v);   // row_mirror
-}
-// LDS words written before by a wave's lanes, read after by its others
-__device__ __forceinline__ void wave_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 // The workgroup's waves meet with their LDS words written and read.  Only the
 // ring passes between the waves of a plane, so nothing waits for the stores to
