@@ -1527,6 +1527,13 @@ struct Prof {
 namespace {
 
 const int kBlock = 256;
+// Workgroup of the stage launches until cs_autotune chooses: one wavefront.
+// They hold no LDS tile, so nothing is shared in a larger one, and single
+// waves spread a small grid over all CUs and refill a large one wave by wave.
+// A step at 256 -> 64 threads: surface 32^2 132 -> 127 us, shells 12^2x4
+// 214 -> 197, 24^2x8 259 -> 238, 95^2x33 3325 -> 3247 (mixed 2916 -> 2796),
+// 160^2x48 12.76 -> 12.52 ms, surface 512^2 1861 -> 1817 us.
+const int kStageBlock = 64;
 inline unsigned nblk(uint64_t n) { return (unsigned)((n + kBlock - 1) / kBlock); }
 inline unsigned nblk_b(uint64_t n, int bs) { return (unsigned)((n + bs - 1) / bs); }
 
@@ -1973,7 +1980,8 @@ extern "C" int cs_create(const cs_config* cfg, cs_handle** out) {
     return CS_E_HIP;
   }
   cs_handle* h = new cs_handle();
-  for (int q = 0; q < CS_K_COUNT; ++q) h->bs[q] = kBlock;
+  for (int q = 0; q < CS_K_COUNT; ++q)  // those without a choice run at kBlock
+    h->bs[q] = q == CS_K_PRIMS || q == CS_K_CLEANUP || q == CS_K_SYNC || q == CS_K_CFL ? kBlock : kStageBlock;
   h->cfg = *cfg;
   h->d = cs_make_dims(cfg->ntp, cfg->nr, cfg->nghost);
   h->pr = Params{cfg->gamma, cfg->gamma - 1.0, cfg->rhofloor, cfg->prsfloor, cfg->cfl, cfg->grav,
@@ -2834,7 +2842,7 @@ extern "C" int cs_batch_create(const cs_config* cfgs, int32_t n, cs_batch** out)
       rc = CS_E_NOMEM;
       break;
     }
-    rc = batch_offsets(B, q, kBlock);
+    rc = batch_offsets(B, q, q == BP_CFL ? kBlock : kStageBlock);
   }
   if (rc) {
     batch_free(B);
