@@ -413,10 +413,13 @@ __device__ __forceinline__ void solve_face(const R* VL, const R* VR, const doubl
 // ------------------------------------------------------------------ face fluxes
 // DIR 0: x-faces (x-vertex i, cells i and i+1), 1: y, 2: z.
 // Output per face: flux(9) * area in the global frame, speeds SL, SR.
-template <int DIR, typename R, typename P>
+// PAIR: the face has two adjacent lanes; lane `side` reconstructs the state on
+// its own side (the right state is the left one's stencil read backwards),
+// the two exchange them and the even lane stores.
+template <int DIR, typename R, typename P, bool PAIR = false>
 __device__ __forceinline__ void face_flux(const CsDims& d, int i, int j, int k, int s, const Geo& geo,
                                           const State& st, const P* __restrict__ V, double* __restrict__ F,
-                                          double* __restrict__ S, const Params& pr) {
+                                          double* __restrict__ S, const Params& pr, int side = 0) {
   if (DIR == 2 && (i == 0 || i == d.N + 1) && (j == 0 || j == d.N + 1)) {
     // radial faces of the tri-corner ghost columns have zero area (two of the
     // four vertices coincide); nothing reads them
@@ -438,7 +441,21 @@ __device__ __forceinline__ void face_flux(const CsDims& d, int i, int j, int k, 
                     (DIR == 0 ? (j >= 1 && j <= d.N)
                               : DIR == 1 ? (i >= 1 && i <= d.N) : (i >= 1 && i <= d.N && j >= 1 && j <= d.N));
   R VL[9], VR[9];
-  for (int q = 0; q < 9; ++q) {
+  if (PAIR) {
+    const int64_t c1 = side ? cl + stride : cl, st1 = side ? -stride : stride;
+    R W[9];
+    for (int q = 0; q < 9; ++q) {
+      const P* p = Vs + q * d.cpp + c1;
+      W[q] = weno ? weno5<R>((R)p[-2 * st1], (R)p[-st1], (R)p[0], (R)p[st1], (R)p[2 * st1]) : (R)p[0];
+    }
+    if (!(W[0] > R(0)) || !(W[4] > R(0)) || !(W[8] > R(0)))
+      for (int q = 0; q < 9; ++q) W[q] = (R)Vs[q * d.cpp + c1];
+    for (int q = 0; q < 9; ++q) {
+      const R o = __shfl_xor(W[q], 1, 64);
+      VL[q] = side ? o : W[q];
+      VR[q] = side ? W[q] : o;
+    }
+  } else for (int q = 0; q < 9; ++q) {
     const P* p = Vs + q * d.cpp + cl;
     if (weno) {
       R m2 = (R)p[-2 * stride], m1 = (R)p[-stride], c0 = (R)p[0], p1 = (R)p[stride],
@@ -450,9 +467,9 @@ __device__ __forceinline__ void face_flux(const CsDims& d, int i, int j, int k, 
       VR[q] = (R)p[stride];
     }
   }
-  if (!(VL[0] > R(0)) || !(VL[4] > R(0)) || !(VL[8] > R(0)))
+  if (!PAIR && (!(VL[0] > R(0)) || !(VL[4] > R(0)) || !(VL[8] > R(0))))
     for (int q = 0; q < 9; ++q) VL[q] = (R)Vs[q * d.cpp + cl];
-  if (!(VR[0] > R(0)) || !(VR[4] > R(0)) || !(VR[8] > R(0)))
+  if (!PAIR && (!(VR[0] > R(0)) || !(VR[4] > R(0)) || !(VR[8] > R(0))))
     for (int q = 0; q < 9; ++q) VR[q] = (R)Vs[q * d.cpp + cl + stride];
   // face frame (A normal, B, C) and area
   double A[3], Bv[3], Cv[3], area, bface;
@@ -486,6 +503,7 @@ __device__ __forceinline__ void face_flux(const CsDims& d, int i, int j, int k, 
   double out[9];
   R SL, SR;
   solve_face<R>(VL, VR, A, Bv, Cv, bface, pr, out, SL, SR);
+  if (PAIR && side) return;
   int64_t fo = (int64_t)s * 9 * d.fpp + d.face(i, j, k);
   for (int q = 0; q < 9; ++q) F[fo + q * d.fpp] = out[q] * area;
   int64_t so = (int64_t)s * 2 * d.fpp + d.face(i, j, k);
@@ -502,18 +520,19 @@ __global__ void __launch_bounds__(256, 2) k_face_flux(CsDims d, Rng rg, Geo geo,
 }
 
 // x- and y-faces of a stage in one launch (the two sweeps are independent)
-template <typename R, typename P>
+template <typename R, typename P, bool PAIR>
 __global__ void __launch_bounds__(256, 2) k_face_flux_xy(CsDims d, Rng rx, Rng ry, Geo geo, State st,
                                                          const P* __restrict__ V, double* __restrict__ Fx,
                                                          double* __restrict__ Sx, double* __restrict__ Fy,
                                                          double* __restrict__ Sy, Params pr) {
-  const uint32_t t = gtid();
+  const uint32_t t = PAIR ? gtid() >> 1 : gtid();
+  const int side = PAIR ? (int)(threadIdx.x & 1) : 0;
   int i, j, k, s;
   if (t < rx.total) {
     decode(rx, t, i, j, k, s);
-    face_flux<0, R, P>(d, i, j, k, s, geo, st, V, Fx, Sx, pr);
+    face_flux<0, R, P, PAIR>(d, i, j, k, s, geo, st, V, Fx, Sx, pr, side);
   } else if (decode(ry, t - rx.total, i, j, k, s)) {
-    face_flux<1, R, P>(d, i, j, k, s, geo, st, V, Fy, Sy, pr);
+    face_flux<1, R, P, PAIR>(d, i, j, k, s, geo, st, V, Fy, Sy, pr, side);
   }
 }
 
@@ -1084,13 +1103,15 @@ __global__ void __launch_bounds__(256, 2) k_update_cells(CsDims d, Rng rg, Geo g
 // are functions of the zone alone.  They are evaluated here, with exactly the
 // reconstruction and Riemann solve k_face_flux<2> applies to that column, and
 // neither the radial ghost fill nor the z-face pass is needed.
-template <typename R, typename P>
+// PAIR: a zone has two adjacent lanes, each solves one of the wall faces.
+template <typename R, typename P, bool PAIR>
 __global__ void __launch_bounds__(256, 2) k_update_cells_surf(CsDims d, Rng rg, Geo geo, State in, State u0, State out,
                                     P* V, const double* __restrict__ Fx,
                                     const double* __restrict__ Fy, const double* dtp, double wa,
                                     double wb, Params pr, int* flags, int mode) {
   int i, j, k, s;
-  if (!decode(rg, gtid(), i, j, k, s)) return;
+  const int side = PAIR ? (int)(threadIdx.x & 1) : 0;
+  if (!decode(rg, PAIR ? gtid() >> 1 : gtid(), i, j, k, s)) return;
   const double dt = dtp[0];
   const int64_t c = d.cell(i, j, k);
   const double r1 = geo.r(d, k), r0 = geo.r(d, k - 1);
@@ -1135,13 +1156,32 @@ __global__ void __launch_bounds__(256, 2) k_update_cells_surf(CsDims d, Rng rg, 
   const bool okp = (Wp[0] > R(0)) && (Wp[4] > R(0)) && (Wp[8] > R(0));
   const bool okm = (Wm[0] > R(0)) && (Wm[4] > R(0)) && (Wm[8] > R(0));
   const int64_t so = (int64_t)s * d.fpp;
-  double fo[9], fi[9];
   R sl, sr;
-  solve_face<R>(okp ? Wp : Vc, okm ? Wm : Vm, A, Bv, Cv, in.Bz[so + d.face(i, j, k)], pr, fo, sl, sr);
-  solve_face<R>(okm ? Wm : Vm, okp ? Wp : Vc, A, Bv, Cv, in.Bz[so + d.face(i, j, k - 1)], pr, fi, sl, sr);
   const double a1 = r1 * r1 * zn, a0 = r0 * r0 * zn;
-  for (int q = 0; q < 9; ++q)
-    if (q < 5 || q == 8) L[q] -= ov * (fo[q] * a1 - fi[q] * a0);
+  if (PAIR) {
+    // the even lane solves the outer wall (zone | ghost), the odd one the inner (ghost | zone)
+    R VL[9], VR[9];
+    for (int q = 0; q < 9; ++q) {
+      const R p = okp ? Wp[q] : Vc[q], m = okm ? Wm[q] : Vm[q];
+      VL[q] = side ? m : p;
+      VR[q] = side ? p : m;
+    }
+    double f[9];
+    solve_face<R>(VL, VR, A, Bv, Cv, in.Bz[so + d.face(i, j, k - side)], pr, f, sl, sr);
+    for (int q = 0; q < 9; ++q)
+      if (q < 5 || q == 8) {
+        const double fi = __shfl_xor(f[q], 1, 64);
+        L[q] -= ov * (f[q] * a1 - fi * a0);
+      }
+    // both lanes have read the zone's V, and the exchange orders that before the stores below
+    if (side) return;
+  } else {
+    double fo[9], fi[9];
+    solve_face<R>(okp ? Wp : Vc, okm ? Wm : Vm, A, Bv, Cv, in.Bz[so + d.face(i, j, k)], pr, fo, sl, sr);
+    solve_face<R>(okm ? Wm : Vm, okp ? Wp : Vc, A, Bv, Cv, in.Bz[so + d.face(i, j, k - 1)], pr, fi, sl, sr);
+    for (int q = 0; q < 9; ++q)
+      if (q < 5 || q == 8) L[q] -= ov * (fo[q] * a1 - fi[q] * a0);
+  }
   const double rcz = 0.5 * (r0 + r1), gr = pr.grav != 0.0 ? -pr.grav / (rcz * rcz) : 0.0;
   if (pr.rot) {
     const double rp[3] = {rcz * A[0], rcz * A[1], rcz * A[2]};
@@ -1658,6 +1698,16 @@ int launch_sync(cs_handle* h, bool flux, bool edge) {
   return CS_OK;
 }
 
+// Surface mode: two lanes a face or zone (PAIR) while that leaves every SIMD at most one
+// wave, 2 n <= 256 CUs x 4 SIMDs x 64 lanes: such a launch is one chain of
+// reconstruction and Riemann solve, and the pair halves the part that the two
+// sides do not share.  A step of a surface, one lane -> two: 16^2 145 -> 122 us,
+// 32^2 131 -> 125, 64^2 (zones only) 152 -> 144; past the line the lanes' shared
+// part costs more than the idle SIMDs give: 96^2 176 -> 190, 128^2 215 -> 249.
+// Shells keep one lane (12^2 x 4 would gain 4 %, 24^2 x 8 nothing): k_batch's
+// one-lane form must give a shell the same bits.
+inline bool lane_pairs(uint64_t n) { return n <= 256 * 4 * 64 / 2; }
+
 // Launch one kernel of the stage on buffer b (update kernels use irk).
 template <typename R, typename P>
 int launch_kernel_t(cs_handle* h, int kid, int b, int irk, bool surf, int halo) {
@@ -1692,8 +1742,12 @@ int launch_kernel_t(cs_handle* h, int kid, int b, int irk, bool surf, int halo) 
       k_face_flux<2, R, P><<<nblk_b(r.fz.total, K), K, 0, sm>>>(d, r.fz, geo, st, V, h->F[2], h->S[2], h->pr);
       break;
     case CS_K_FLUX_XY:
-      k_face_flux_xy<R, P><<<nblk_b((uint64_t)r.fx.total + r.fy.total, K), K, 0, sm>>>(
-          d, r.fx, r.fy, geo, st, V, h->F[0], h->S[0], h->F[1], h->S[1], h->pr);
+      if (surf && lane_pairs((uint64_t)r.fx.total + r.fy.total))
+        k_face_flux_xy<R, P, true><<<nblk_b(2 * ((uint64_t)r.fx.total + r.fy.total), K), K, 0, sm>>>(
+            d, r.fx, r.fy, geo, st, V, h->F[0], h->S[0], h->F[1], h->S[1], h->pr);
+      else
+        k_face_flux_xy<R, P, false><<<nblk_b((uint64_t)r.fx.total + r.fy.total, K), K, 0, sm>>>(
+            d, r.fx, r.fy, geo, st, V, h->F[0], h->S[0], h->F[1], h->S[1], h->pr);
       break;
     case CS_K_EMF:
       k_emf_all<P><<<nblk_b((uint64_t)r.ez.total + r.ex.total + r.ey.total, K), K, 0, sm>>>(
@@ -1709,10 +1763,14 @@ int launch_kernel_t(cs_handle* h, int kid, int b, int irk, bool surf, int halo) 
       if (r.ey.total) k_emf_xy<1, P><<<nblk_b(r.ey.total, K), K, 0, sm>>>(d, r.ey, geo, st, V, h->S[2], h->S[0], h->E[1], h->pr);
       break;
     case CS_K_UPDATE_CELLS:  // zone update + cleanup + primitives of the output
-      if (surf)
-        k_update_cells_surf<R, P><<<nblk_b(r.cells.total, K), K, 0, sm>>>(d, r.cells, geo, in, u0, out, V, h->F[0],
-                                                                          h->F[1], h->dt, wa, wb, h->pr, h->flags,
-                                                                          h->pr.imex ? irk : 0);
+      if (surf && lane_pairs(r.cells.total))
+        k_update_cells_surf<R, P, true><<<nblk_b(2 * (uint64_t)r.cells.total, K), K, 0, sm>>>(
+            d, r.cells, geo, in, u0, out, V, h->F[0], h->F[1], h->dt, wa, wb, h->pr, h->flags,
+            h->pr.imex ? irk : 0);
+      else if (surf)
+        k_update_cells_surf<R, P, false><<<nblk_b(r.cells.total, K), K, 0, sm>>>(
+            d, r.cells, geo, in, u0, out, V, h->F[0], h->F[1], h->dt, wa, wb, h->pr, h->flags,
+            h->pr.imex ? irk : 0);
       else
         k_update_cells<P><<<nblk_b(r.cells.total, K), K, 0, sm>>>(d, r.cells, geo, in, u0, out, h->F[0], h->F[1],
                                                                     h->F[2], h->dt, wa, wb, h->pr, V, h->flags,
