@@ -53,7 +53,8 @@ void set_error(const char* fmt, ...);
 namespace p1s {
 
 constexpr int kSweeps = 12;          // bound on the positivity replay sweeps per stage
-constexpr int kListBlocks = 512;     // grid of the replay kernels (grid-stride)
+constexpr int kListBlocks = 512;     // grid of k_replay and k_clear_ent (grid-stride)
+constexpr int kCandBlocks = 2048;    // largest grid of k_cands (grid-stride)
 constexpr int kCflBlocks = 1024;     // grid of the time-step reduction
 // counters: [0] zones whose slopes pass 0 removed, [1] list length,
 // [2 .. 2 + kSweeps) flag changes per sweep
@@ -732,8 +733,8 @@ __device__ __forceinline__ bool replay_done(const Dev& D, int sweep) {
 // among their 27 join the list (each once: the list only grows, so a zone
 // that depends on a flag is recomputed in every later sweep; both flag
 // arrays of a zone that joins still hold its first pass's flag).
-// Grid-stride over the six sectors: an idle sweep costs a small launch
-// whatever the shell's size.
+// Grid-stride over the six sectors, eight waves a SIMD at most: an idle sweep
+// costs a small launch whatever the shell's size.
 __global__ void __launch_bounds__(256) k_cands(Dev D, Box b, int sweep) {
   if (replay_done(D, sweep)) return;
   const int64_t n = b.count(), ks = (int64_t)D.nz * D.nz;
@@ -758,18 +759,23 @@ __global__ void __launch_bounds__(256) k_cands(Dev D, Box b, int sweep) {
     }
   }
 }
-// the list's zones in groups of 64: three waves redo their WENO (three fields
-// each), then the first wave their positivity.  The replay was 48 launches a
-// stage (candidates, WENO, positivity and the flags' commit in each of the 12
-// sweeps) and is 24 small ones.  Idle, it costs their latency: 24^2 x 8
-// 81 -> 43 us, 160^2 x 48 180 -> 46 us; the 256^2 blast surface, where it
-// has zones to redo, 107 -> 78 us.
-constexpr int kReplayZones = 64;
-__global__ void __launch_bounds__(3 * kReplayZones) k_replay(Dev D, int sweep) {
+// the list's zones: WENO again, then positivity.  A list that gives every
+// workgroup one group of 64 zones at most is latency: three waves take the
+// zones' fields, three each, then the first wave their positivity.  A longer
+// one is throughput: a lane does both for its zone, so that all four waves
+// work on positivity.  Two waves per SIMD (249 registers; without the bound
+// the compiler takes 270 and one).  A step with log-normal noise of 0.8 on the
+// density, three-wave form alone -> both: 96^2 x 32 65.0 -> 28.3 ms, 256^2
+// surface 57.0 -> 31.3 ms, 45^2 x 17 7.8 -> 4.2 ms.  Idle, a stage's 24 launches
+// cost their latency, some 45 us whatever the shell's size (81 us at 24^2 x 8 and
+// 180 at 160^2 x 48 for four launches a sweep over full grids).
+constexpr int kReplayZones = 64, kReplayThreads = 256;
+__global__ void __attribute__((amdgpu_waves_per_eu(2))) __launch_bounds__(kReplayThreads) k_replay(Dev D, int sweep) {
   if (replay_done(D, sweep)) return;
   const int64_t n = D.ctr[1];
-  const int q = threadIdx.x % kReplayZones, grp = threadIdx.x / kReplayZones;
-  for (int64_t t0 = (int64_t)blockIdx.x * kReplayZones; t0 < n; t0 += (int64_t)gridDim.x * kReplayZones) {
+  const int nzb = n <= (int64_t)gridDim.x * kReplayZones ? kReplayZones : kReplayThreads;
+  const int q = threadIdx.x % nzb, grp = threadIdx.x / nzb;
+  for (int64_t t0 = (int64_t)blockIdx.x * nzb; t0 < n; t0 += (int64_t)gridDim.x * nzb) {
     const bool on = t0 + q < n;
     int s = 0, i = 0, j = 0, k = 0;
     int64_t z = 0;
@@ -778,7 +784,8 @@ __global__ void __launch_bounds__(3 * kReplayZones) k_replay(Dev D, int sweep) {
       s = (int)(p / D.NZ);
       z = p - (int64_t)s * D.NZ;
       D.zone_of(z, i, j, k);
-      weno3(D, s, i, j, k, z, 3 * grp);
+#pragma unroll 1
+      for (int c = grp; c < 3; c += kReplayThreads / nzb) weno3(D, s, i, j, k, z, 3 * c);
     }
     __syncthreads();  // the zone's slopes are written before its positivity reads them
     if (on && grp == 0) positivity(D, s, i, j, k, z, sweep);
@@ -2180,8 +2187,8 @@ int front(Stage* S, const Buf& in_, double* const* F, double* const* Sp, double*
   mark_end(S, st, CS_P1K_POSITIVITY);
   mark_begin(S, st);
   for (int sw = 0; sw < kSweeps; ++sw) {
-    k_cands<<<kListBlocks, 256, 0, st>>>(D, S->wr, sw);
-    k_replay<<<kListBlocks, 3 * kReplayZones, 0, st>>>(D, sw);
+    k_cands<<<std::min<unsigned>(kCandBlocks, nb(6 * nwr, 256)), 256, 0, st>>>(D, S->wr, sw);
+    k_replay<<<kListBlocks, kReplayThreads, 0, st>>>(D, sw);
   }
   k_clear_ent<<<kListBlocks, 256, 0, st>>>(D, S->wr, in, err);
   mark_end(S, st, CS_P1K_REPLAY);

@@ -699,7 +699,8 @@ __global__ void __attribute__((amdgpu_waves_per_eu(2))) __launch_bounds__(256)
 // the list only grows, so a zone whose result depends on a flag is
 // recomputed in every later sweep; a zone that joins has its first pass's
 // flag in both arrays)
-constexpr int kListBlocks = 512;  // grids of the replay kernels (grid-stride)
+constexpr int kListBlocks = 512;   // grids of the list's kernels at 256 threads (grid-stride)
+constexpr int kCandBlocks = 2048;  // largest grid of k_cands (grid-stride)
 __global__ void __launch_bounds__(256) k_cands(const P1 P, const Box b, const Flags F, int sweep) {
   if (F.done(sweep)) return;
   const int64_t n = b.count(), ks = (int64_t)P.nz * P.nz;
@@ -723,25 +724,30 @@ __global__ void __launch_bounds__(256) k_cands(const P1 P, const Box b, const Fl
     }
   }
 }
-// one sweep over the list in groups of 64 zones: three waves redo their WENO
-// (three fields each), then the first wave their positivity.  The counts and
-// the flags stay on the device, so the host looks once per kSweepBatch sweeps
-// instead of twice per sweep (the call on a noisy 16^2 x 6 patch 423 -> 370 us,
-// 128^2 x 48 2.42 -> 2.29 ms)
-constexpr int kReplayZones = 64;
-__global__ void __attribute__((amdgpu_waves_per_eu(2))) __launch_bounds__(3 * kReplayZones)
+// one sweep over the list: WENO again, then positivity.  A list that gives
+// every workgroup one group of 64 zones at most is latency: three waves take
+// the zones' fields, three each, then the first wave their positivity.  A
+// longer one is throughput: a lane does both for its zone, so that all four
+// waves work on positivity (192^2 x 64 with noise of 1.0 on the density 27.6 ->
+// 14.8 ms a call, 128^2 x 48 with 1.5 7.8 -> 4.5).  The counts and the flags stay on the device, so
+// the host looks once per kSweepBatch sweeps instead of twice per sweep (the
+// call on a noisy 16^2 x 6 patch 423 -> 370 us, 128^2 x 48 2.42 -> 2.29 ms)
+constexpr int kReplayZones = 64, kReplayThreads = 256;
+__global__ void __attribute__((amdgpu_waves_per_eu(2))) __launch_bounds__(kReplayThreads)
     k_replay(const P1 P, const Flags F, const WenoFields W9, int sweep) {
   if (F.done(sweep)) return;
   const int64_t n = F.ctr[1];
-  const int q = threadIdx.x % kReplayZones, grp = threadIdx.x / kReplayZones;
-  for (int64_t t0 = (int64_t)blockIdx.x * kReplayZones; t0 < n; t0 += (int64_t)gridDim.x * kReplayZones) {
+  const int nzb = n <= (int64_t)gridDim.x * kReplayZones ? kReplayZones : kReplayThreads;
+  const int q = threadIdx.x % nzb, grp = threadIdx.x / nzb;
+  for (int64_t t0 = (int64_t)blockIdx.x * nzb; t0 < n; t0 += (int64_t)gridDim.x * nzb) {
     const bool on = t0 + q < n;
     int i = 0, j = 0, k = 0;
     int64_t z = 0;
     if (on) {
       z = F.list[t0 + q];
       zone_of(P, z, i, j, k);
-      weno_group(P, i, j, k, z, 3 * grp, W9);
+#pragma unroll 1
+      for (int c = grp; c < 3; c += kReplayThreads / nzb) weno_group(P, i, j, k, z, 3 * c, W9);
     }
     __syncthreads();  // the zone's slopes are written before its positivity reads them
     if (on && grp == 0) pos_zone<4>(P, i, j, k, z, sweep, F, nullptr);
@@ -1287,13 +1293,13 @@ static int run_p1(const cs_p1_patch* p, void* stream_, float* kernel_ms, uint8_t
     unsigned int nchg = 1;
     for (int sw = 0; sw < kMaxSweeps && nchg > 0;) {
       for (int q = 0; q < kSweepBatch; ++q, ++sw) {
-        k_cands<<<kListBlocks, 256, 0, st>>>(P, wr, F, sw);
+        k_cands<<<std::min<unsigned>(kCandBlocks, grid_of(wr.count(), 256)), 256, 0, st>>>(P, wr, F, sw);
         if (mom) {
-          k_weno9_list<<<kListBlocks, 128, 0, st>>>(P, F, wv, sw);
-          k_weno_ao_list<<<kListBlocks, 128, 0, st>>>(P, ao, mom, F, sw);
+          k_weno9_list<<<2 * kListBlocks, 128, 0, st>>>(P, F, wv, sw);
+          k_weno_ao_list<<<2 * kListBlocks, 128, 0, st>>>(P, ao, mom, F, sw);
           k_pos10_list<<<kListBlocks, 256, 0, st>>>(P, F, mom, sw);
         } else {
-          k_replay<<<kListBlocks, 3 * kReplayZones, 0, st>>>(P, F, wv, sw);
+          k_replay<<<kListBlocks, kReplayThreads, 0, st>>>(P, F, wv, sw);
         }
       }
       P1_HIP(hipGetLastError());

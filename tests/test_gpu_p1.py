@@ -79,6 +79,34 @@ def test_p1_gpu_matches_oracle(case):
     np.testing.assert_array_equal(np.abs(vg[1:, :5]).sum((0, 1)) == 0, np.abs(vo[1:, :5]).sum((0, 1)) == 0)
 
 
+def later_neighbours(flag):
+    """The zones with a flagged zone earlier in the loop order among their 27
+    (two layers off the array's sides, where the limiter works; no tri-corner re-pointing): a lower bound of the
+    replay list's length."""
+    c = np.zeros_like(flag)
+    for dk in (-1, 0, 1):
+        for dj in (-1, 0, 1):
+            for di in (-1, 0, 1):
+                if (dk, dj, di) < (0, 0, 0):
+                    c |= np.roll(flag, (-dk, -dj, -di), (-3, -2, -1))
+    return int(c[..., 2:-2, 2:-2, 2:-2].sum())
+
+
+def test_p1_gpu_long_replay_list_matches_oracle():
+    """More zones on the positivity replay's list than its 512 workgroups take
+    in groups of 64: a lane then redoes all fields of its zone."""
+    N, NR = 48, 20
+    print("p1 case long replay list", flush=True)
+    prob, A0 = orc.p1_problem(N, NR, 4, sector=1, seed=6, shock=True, noise=1.5)
+    O = orc.p1_oracle(prob, orc.p1_copy(A0))
+    assert later_neighbours(O["ent"].reshape(4, NR + 8, N + 8, N + 8)[0] == 0) > 512 * 64
+    G = _run_gpu(prob, orc.p1_copy(A0))
+    bad = _compare(G, {k: O[k] for k in G})
+    assert not bad, bad
+    nz = orc.p1_dims(N, NR, 4)["zone"]
+    np.testing.assert_array_equal(G["ent"].reshape(4, nz)[0] == 0, O["ent"].reshape(4, nz)[0] == 0)
+
+
 def test_p1_gpu_rejects_bad_sizes():
     prob, A = orc.p1_problem(8, 3, 4)
     dev = torch.device("cuda:0")

@@ -31,6 +31,7 @@ import pytest
 
 import cubesphere_amd as cs
 from oracle import oracle as orc
+from test_gpu_p1 import later_neighbours
 
 pytestmark = pytest.mark.gpu
 
@@ -190,6 +191,33 @@ def test_p1_stage_march_chunks():
     finally:
         h.close()
     _compare(cfg, got, ref, 1e-9)
+
+
+def test_p1_stage_long_replay_list():
+    """The positivity replay with more zones on its list than its 512
+    workgroups take in groups of 64 (a lane then redoes all fields of its
+    zone): one step on a shell whose noise removes the slopes of a tenth of the
+    zones, against the oracle."""
+    cfg = cs.make_config(24, 20, 4, cs.RECON_P1ADP, cs.RS_HLLD, cs.EMF_LLF, cs.FP64, 2, cs.RBC_PAD, cs.RMESH_UNIFORM,
+                         1.0, 1.5)
+    st0 = _state(cfg, 2, 1.5)
+    ref = st0.copy()
+    print("long replay list: oracle step", flush=True)
+    As = orc.p1s_patches(cfg)
+    dt1 = orc.p1s_step_oracle(orc.Grid(cfg), cfg, As, ref, 2e-5)
+    print("long replay list: device step", flush=True)
+    h = cs.CubeSphere(cfg)
+    try:
+        h.upload(st0)
+        h.dt = 2e-5
+        h.advance(1)
+        got = h.download()
+        assert abs(h.dt - dt1) <= 1e-9 * dt1
+    finally:
+        h.close()
+    _compare(cfg, got, ref, 1e-9)
+    gone = np.array([A["ent"].reshape(4, 28, 32, 32)[0] == 0.0 for A in As])  # the last stage's removed zones
+    assert later_neighbours(gone) > 512 * 64
 
 
 def test_p1_stage_graph_equals_eager():
