@@ -45,15 +45,20 @@ struct Staging {
   char* pin = nullptr;
   int device = -1;
   hipEvent_t ev[kSlots] = {};
+  // for streams of device dev, whichever is the calling thread's: an event can
+  // only be recorded on a stream of the device that was current when it was made
   bool make(int dev) {
     device = dev;
-    bool ok = hipHostMalloc((void**)&pin, kSlots * kSlotMax, hipHostMallocDefault) == hipSuccess;
+    int was = dev;
+    bool ok = hipGetDevice(&was) == hipSuccess && (was == dev || hipSetDevice(dev) == hipSuccess);
+    ok = ok && hipHostMalloc((void**)&pin, kSlots * kSlotMax, hipHostMallocDefault) == hipSuccess;
     if (!ok) pin = nullptr;
     for (hipEvent_t& e : ev)
       if (ok && hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) {
         e = nullptr;
         ok = false;
       }
+    if (was != dev) (void)hipSetDevice(was);
     if (!ok) (void)hipGetLastError();
     return ok;
   }
@@ -80,9 +85,12 @@ class StagingPool {
     if (--handles_ == 0)
       for (size_t q = 0; q < kIdleSets; ++q) drop[q] = std::move(idle_[q]);
   }
-  std::unique_ptr<Staging> take() {
+  std::unique_ptr<Staging> take(hipStream_t st) {
     int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess) return nullptr;
+    if (hipStreamGetDevice(st, &dev) != hipSuccess) {
+      (void)hipGetLastError();
+      return nullptr;
+    }
     {
       std::lock_guard<std::mutex> l(mu_);
       for (auto& s : idle_)
@@ -196,7 +204,7 @@ inline hipError_t transfer(hipStream_t st, const Segment* seg, int nseg, bool to
   size_t total = 0;
   for (int q = 0; q < nseg; ++q) total += seg[q].bytes;
   std::unique_ptr<Staging> S;
-  if (total >= (to_host ? kStagedDown : kStagedUp)) S = staging_pool().take();
+  if (total >= (to_host ? kStagedDown : kStagedUp)) S = staging_pool().take(st);
   if (S) {
     Transfer T(seg, nseg, total, *S, to_host);
     std::thread th[kWorkers];

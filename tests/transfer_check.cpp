@@ -1,0 +1,79 @@
+// Host check of the state transfers' staging (cs_transfer.h) over the fake
+// runtime of fake_hip/: argument 1 names the check, "ok" is printed when it holds.
+#include "cs_transfer.h"
+
+#include <stdio.h>
+
+#include <string>
+#include <vector>
+
+using namespace cs;
+
+static int fail(const char* what) {
+  printf("%s\n", what);
+  return 1;
+}
+
+// a state in three arrays of uneven size, past the threshold of its direction
+struct State {
+  std::vector<char> dev[3], host[3];
+  Segment seg[3];
+  explicit State(size_t mib) {
+    const size_t n[3] = {(mib << 19) + 24, (mib << 18) + 8, (mib << 18) + 4096};
+    for (int q = 0; q < 3; ++q) {
+      dev[q].resize(n[q]);
+      host[q].resize(n[q]);
+      seg[q] = Segment{dev[q].data(), host[q].data(), n[q]};
+    }
+  }
+  size_t bytes() const { return dev[0].size() + dev[1].size() + dev[2].size(); }
+  void fill(bool down, int seed) {
+    for (int q = 0; q < 3; ++q) {
+      auto &a = down ? dev[q] : host[q], &b = down ? host[q] : dev[q];
+      for (size_t i = 0; i < a.size(); ++i) a[i] = (char)((i * 2654435761u + seed) >> 7);
+      std::fill(b.begin(), b.end(), 0);
+    }
+  }
+  bool same() const { return dev[0] == host[0] && dev[1] == host[1] && dev[2] == host[2]; }
+};
+
+// the handle's stream on a device that is not the calling thread's
+static int other_device() {
+  FakeStream st{1};
+  for (bool down : {true, false}) {
+    State S(down ? 25 : 66);
+    S.fill(down, 3);
+    fake().direct = fake().staged = 0;
+    if (transfer(&st, S.seg, 3, down) != hipSuccess) return fail("a transfer of a handle on another device failed");
+    if (!S.same()) return fail("words lost");
+    if (fake().staged != S.bytes()) return fail("not staged");
+    if (fake().device != 0) return fail("the calling thread's device was changed");
+  }
+  return 0;
+}
+
+// staging that fails half way: the plain copies take over, and no error is left behind
+static int fall_back() {
+  FakeStream st{0};
+  for (bool down : {true, false}) {
+    State S(down ? 40 : 80);
+    S.fill(down, 5);
+    fake().fail_record = 1;
+    if (transfer(&st, S.seg, 3, down) != hipSuccess) return fail("no fall back to the plain copies");
+    if (!S.same()) return fail("words lost");
+    if (hipGetLastError() != hipSuccess) return fail("an error is left for the next call");
+  }
+  return 0;
+}
+
+int main(int argc, char** argv) {
+  const std::string what = argc > 1 ? argv[1] : "";
+  int rc = 2;
+  staging_pool().enter();
+  if (what == "other_device") rc = other_device();
+  if (what == "fall_back") rc = fall_back();
+  staging_pool().leave();
+  if (rc == 0 && (fake().events != 0 || !fake().pin.empty())) rc = fail("slots kept after the last handle");
+  if (rc == 0) printf("ok\n");
+  return rc;
+}
