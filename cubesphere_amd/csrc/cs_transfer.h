@@ -198,8 +198,8 @@ struct Transfer {
 };
 
 // Copies the segments on `st` and waits for them.  Staged down from 24 MiB and
-// up from 64 MiB; below, and where no slots or threads are to be had, the
-// runtime's copies.
+// up from 64 MiB; below, and where no slots or threads are to be had or the
+// staging fails, the runtime's copies.
 inline hipError_t transfer(hipStream_t st, const Segment* seg, int nseg, bool to_host) {
   size_t total = 0;
   for (int q = 0; q < nseg; ++q) total += seg[q].bytes;
@@ -219,9 +219,11 @@ inline hipError_t transfer(hipStream_t st, const Segment* seg, int nseg, bool to
       const hipError_t e = T.drive(st, S->ev);
       for (int t = 0; t < have; ++t) th[t].join();
       staging_pool().give(std::move(S));
-      return e;
+      if (e == hipSuccess) return e;
+      (void)hipGetLastError();  // the plain copies below redo the whole transfer, and report what still fails
+    } else {
+      staging_pool().give(std::move(S));
     }
-    staging_pool().give(std::move(S));
   }
   for (int q = 0; q < nseg; ++q) {
     const hipError_t e = to_host ? hipMemcpyAsync(seg[q].host, seg[q].dev, seg[q].bytes, hipMemcpyDeviceToHost, st)
