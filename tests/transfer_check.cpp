@@ -66,12 +66,51 @@ static int fall_back() {
   return 0;
 }
 
+// arrays that the runtime can reach by itself: its own copies, no pass through the slots
+static int pinned_arrays() {
+  FakeStream st{0};
+  for (bool down : {true, false})
+    for (int pin = 0; pin < 3; ++pin) {  // none, one, all of them
+      State S(down ? 25 : 66);
+      char* own[3] = {};
+      for (int q = 0; q < 3; ++q)
+        if (pin == 2 || (pin == 1 && q == 1)) {
+          if (hipHostMalloc((void**)&own[q], S.seg[q].bytes / 4096 * 4096 + 4088, hipHostMallocDefault) != hipSuccess)
+            return fail("no memory");
+          S.seg[q].bytes = S.seg[q].bytes / 4096 * 4096;
+          S.seg[q].host = own[q];
+          S.host[q].resize(S.seg[q].bytes);
+          S.dev[q].resize(S.seg[q].bytes);
+          S.seg[q].dev = S.dev[q].data();
+        }
+      S.fill(down, 7);
+      if (!down)
+        for (int q = 0; q < 3; ++q)
+          if (own[q]) memcpy(own[q], S.host[q].data(), S.seg[q].bytes);
+      fake().direct = fake().staged = 0;
+      if (transfer(&st, S.seg, 3, down) != hipSuccess) return fail("failed");
+      size_t direct = 0;
+      for (int q = 0; q < 3; ++q)
+        if (own[q]) {
+          direct += S.seg[q].bytes;
+          if (down) memcpy(S.host[q].data(), own[q], S.seg[q].bytes);
+        }
+      if (!S.same()) return fail("words lost");
+      if (pin == 0 && fake().staged != S.bytes()) return fail("pageable arrays not staged");
+      if (fake().direct < direct) return fail("a pinned array went through the slots");
+      for (char* p : own)
+        if (p) hipHostFree(p);
+    }
+  return 0;
+}
+
 int main(int argc, char** argv) {
   const std::string what = argc > 1 ? argv[1] : "";
   int rc = 2;
   staging_pool().enter();
   if (what == "other_device") rc = other_device();
   if (what == "fall_back") rc = fall_back();
+  if (what == "pinned_arrays") rc = pinned_arrays();
   staging_pool().leave();
   if (rc == 0 && (fake().events != 0 || !fake().pin.empty())) rc = fail("slots kept after the last handle");
   if (rc == 0) printf("ok\n");
