@@ -19,10 +19,10 @@
 
 #include <algorithm>
 #include <atomic>
+#include <exception>
 #include <memory>
 #include <mutex>
 #include <new>
-#include <system_error>
 #include <thread>
 
 namespace cs {
@@ -116,7 +116,8 @@ class StagingPool {
 };
 // never destroyed: the runtime may be gone by the time static objects are
 inline StagingPool& staging_pool() {
-  static StagingPool* p = new StagingPool();
+  alignas(StagingPool) static char mem[sizeof(StagingPool)];
+  static StagingPool* p = new (mem) StagingPool();
   return *p;
 }
 
@@ -239,7 +240,7 @@ inline hipError_t transfer(hipStream_t st, const Segment* all, int nall, bool to
     int have = 0;
     try {
       for (; have < want; ++have) th[have] = std::thread(&Transfer::work, &T);
-    } catch (const std::system_error&) {  // fewer threads share the chunks
+    } catch (const std::exception&) {  // no thread or no memory for its start: fewer share the chunks
     }
     if (have > 0) {
       const hipError_t e = T.drive(st, S->ev);

@@ -3,11 +3,22 @@
 #include "cs_transfer.h"
 
 #include <stdio.h>
+#include <stdlib.h>
 
 #include <string>
 #include <vector>
 
 using namespace cs;
+
+// operator new fails once `budget` more allocations have been made (-1: never)
+static std::atomic<int> budget{-1};
+void* operator new(size_t n) {
+  if (budget.load() >= 0 && budget.fetch_sub(1) <= 0) throw std::bad_alloc();
+  if (void* p = malloc(n)) return p;
+  throw std::bad_alloc();
+}
+void operator delete(void* p) noexcept { free(p); }
+void operator delete(void* p, size_t) noexcept { free(p); }
 
 static int fail(const char* what) {
   printf("%s\n", what);
@@ -104,6 +115,24 @@ static int pinned_arrays() {
   return 0;
 }
 
+// no memory for any thread's start, or after the first or the third (the slots are in the pool)
+static int no_thread_memory() {
+  FakeStream st{0};
+  State warm(25);
+  if (transfer(&st, warm.seg, 3, true) != hipSuccess) return fail("failed");
+  for (bool down : {true, false})
+    for (int have : {0, 1, 3}) {
+      State S(down ? 25 : 66);
+      S.fill(down, 11);
+      budget = have;
+      const hipError_t e = transfer(&st, S.seg, 3, down);
+      budget = -1;
+      if (e != hipSuccess) return fail("failed");
+      if (!S.same()) return fail("words lost");
+    }
+  return 0;
+}
+
 int main(int argc, char** argv) {
   const std::string what = argc > 1 ? argv[1] : "";
   int rc = 2;
@@ -111,6 +140,7 @@ int main(int argc, char** argv) {
   if (what == "other_device") rc = other_device();
   if (what == "fall_back") rc = fall_back();
   if (what == "pinned_arrays") rc = pinned_arrays();
+  if (what == "no_thread_memory") rc = no_thread_memory();
   staging_pool().leave();
   if (rc == 0 && (fake().events != 0 || !fake().pin.empty())) rc = fail("slots kept after the last handle");
   if (rc == 0) printf("ok\n");
