@@ -2771,7 +2771,8 @@ extern "C" int cs_pad_boundary_r_p1(const cs_p1_pad* p, void* stream_) {
 // address modes 1-4, which a ten-mode array lays out exactly as a four-mode
 // one); k_zero_hi clears modes 5-10, k_weno_ao is step 7.b, k_pos<10> 7.c,
 // k_face_pts<10> 8.a-c, k_clsq12 8.d, k_e12 9.a, k_weno9 on E 9.b,
-// k_ao_order / k_ao_e_pre / k_weno_ao_e 9.c, and the P1 diagnostics step 10.
+// k_ao_order / k_ao_e_pre / k_ao_e_sweep / k_ao_e_put 9.c, and the P1
+// diagnostics step 10.
 namespace csp1 {
 
 __global__ void __launch_bounds__(256) k_zero_hi(const P1 P, const Box b) {
@@ -3327,8 +3328,16 @@ constexpr int kAoIx = 160;   // 16 int32: [0..4] box index of each zone below (-
                              // the plane (-1: an inactive zone), [8..15] these (ring slot, or -2 - box index)
 constexpr int kAoGf = 168;   // [4][10]: G for further earlier zones (tri-corner strips)
 // the newest values of each row of a plane in LDS: rows modulo kRingRows, the
-// last kRing zones of a row
-constexpr int kRing = 16, kRingRows = 64;
+// last kRing zones of a row (64 KB; a workgroup of eight waves at two per SIMD
+// fills its CU whatever it holds).  With s levels a row the neighbours at
+// (-1, -1) lie s + 1 levels back and the farthest entry of a panel's own table,
+// at a tri-corner strip, 2 s + 2: kRing covers every entry of patches up to 388
+// zones across (s = 14) and the ordinary ones up to 836 (s = 30).  Those
+// further back come from memory, a round trip in the level's chain: with 16
+// zones a row that began at 389 across for a fourth of the entries, and 392^2 x 1
+// took 23.0 ms for step 9 (17.8 now), 512^2 x 1 47.0 (29.2).  A slot is written again no
+// sooner than s kRingRows - 28 s levels after its row's last zone, more than kRing.
+constexpr int kRing = 32, kRingRows = 64;
 // no result of arithmetic: a signalling NaN marks a point value not yet formed
 constexpr unsigned long long kAoEmpty = 0x7ff0dead0badf00dull;
 
@@ -3565,7 +3574,7 @@ __device__ __forceinline__ bool ao_empty(double v) { return (unsigned long long)
 // bound by the address unit).  A zone's record and the values of the plane
 // below are read two levels ahead, its indices three; the values of the same
 // plane, written in the last levels, come from a ring of the newest values of
-// each row in LDS (a tri-corner zone's entry further back from memory), so
+// each row in LDS (an entry kRing or more levels back from memory), so
 // the chain of a level is: ring, four rows of G, the sum of the indicator
 // over the group, the weights, ring.
 //

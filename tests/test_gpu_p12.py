@@ -47,6 +47,8 @@ CASES = [
     # step 9.c's sweep beyond three levels a row (92 zones across) and past the 64 rows of its ring; a thin
     # shell, so that the zones are not 30 times deeper than wide
     (88, 1, 2, 21, True, 0.3, 4, 1.02),
+    # seven levels a row: entries at the tri-corner strips 16 levels back
+    (168, 1, 1, 23, True, 0.3, 4, 1.02),
 ]
 
 
@@ -111,6 +113,29 @@ def test_p12_rejects_a_stencil_that_breaks_the_step9c_order():
     A["stencil"][s + nz * nz] = 4
     with pytest.raises(cs.CsError, match="level order"):
         _run_gpu(prob, A)
+
+
+def test_p12_entries_far_back_match_oracle():
+    """Step 9.c's sweep keeps the last 32 zones of a row in LDS and reads older
+    values from memory.  A panel's own table needs that from 389 zones across
+    (2 s + 2 levels back, s = 15 levels a row); here (s = 4) some zones' lower
+    diagonal neighbours are moved 8 and 9 rows down, 33 and 35 levels back."""
+    N, NR, g = 88, 1, 4
+    print("case p12 far entries", flush=True)
+    prob, A0 = orc.p12_problem(N, NR, g, sector=3, seed=25, shock=True, noise=0.1, rmax=1.02)
+    nz = N + 2 * g
+    st = A0["stencil"].reshape(12, 2, nz, nz)  # direction, (i, j), at [j][i]
+    for j in (11, 30, 51, 88):
+        for i in (2, 21, 40, 87):
+            jj, ii = j + g - 1, i + g - 1
+            assert tuple(st[10, :, jj, ii]) == (i - 1, j - 1) and tuple(st[11, :, jj, ii]) == (i + 1, j - 1)
+            st[10, 1, jj, ii] = j - 8
+            st[11, 1, jj, ii] = j - 9
+    O = orc.p12_oracle(prob, orc.p1_copy(A0))
+    G = _run_gpu(prob, orc.p1_copy(A0))
+    for k in ("Ex_zc", "Ey_zc", "Ez_zc"):
+        for r, (gr, orow) in enumerate(zip(G[k].reshape(10, -1), O[k].reshape(10, -1))):
+            assert np.abs(gr - orow).max() <= 1e-9 * np.abs(orow).max(), (k, r)
 
 
 def test_p12_timed_matches_untimed():
