@@ -2186,9 +2186,11 @@ int front(Stage* S, const Buf& in_, double* const* F, double* const* Sp, double*
   k_pos<<<dim3(nb(nwr, 256), 6), 256, 0, st>>>(D, S->wr);
   mark_end(S, st, CS_P1K_POSITIVITY);
   mark_begin(S, st);
+  // no more workgroups than a list of the whole range has groups of 64
+  const unsigned nlist = std::min<unsigned>(kListBlocks, nb(6 * nwr, kReplayZones));
   for (int sw = 0; sw < kSweeps; ++sw) {
     k_cands<<<std::min<unsigned>(kCandBlocks, nb(6 * nwr, 256)), 256, 0, st>>>(D, S->wr, sw);
-    k_replay<<<kListBlocks, kReplayThreads, 0, st>>>(D, sw);
+    k_replay<<<nlist, kReplayThreads, 0, st>>>(D, sw);
   }
   k_clear_ent<<<kListBlocks, 256, 0, st>>>(D, S->wr, in, err);
   mark_end(S, st, CS_P1K_REPLAY);

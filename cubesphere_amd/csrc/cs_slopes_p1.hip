@@ -1291,6 +1291,8 @@ static int run_p1(const cs_p1_patch* p, void* stream_, float* kernel_ms, uint8_t
     // flags; a zone newly flagged in a sweep brings its later neighbours
     // onto the list before the next one
     unsigned int nchg = 1;
+    // no more workgroups than a list of the whole range has groups of 64
+    const unsigned nlist = std::min<unsigned>(kListBlocks, grid_of(wr.count(), kReplayZones));
     for (int sw = 0; sw < kMaxSweeps && nchg > 0;) {
       for (int q = 0; q < kSweepBatch; ++q, ++sw) {
         k_cands<<<std::min<unsigned>(kCandBlocks, grid_of(wr.count(), 256)), 256, 0, st>>>(P, wr, F, sw);
@@ -1299,7 +1301,7 @@ static int run_p1(const cs_p1_patch* p, void* stream_, float* kernel_ms, uint8_t
           k_weno_ao_list<<<2 * kListBlocks, 128, 0, st>>>(P, ao, mom, F, sw);
           k_pos10_list<<<kListBlocks, 256, 0, st>>>(P, F, mom, sw);
         } else {
-          k_replay<<<kListBlocks, kReplayThreads, 0, st>>>(P, F, wv, sw);
+          k_replay<<<nlist, kReplayThreads, 0, st>>>(P, F, wv, sw);
         }
       }
       P1_HIP(hipGetLastError());
