@@ -3275,7 +3275,9 @@ __global__ void __launch_bounds__(256) k_e12(const P1 P, const Box b, const doub
 // differs by at most 2 in i, so a row step of 3 outweighs it, and a neighbour
 // above or below by at most 2 + 3 * 2 = 8 within the plane, which a plane step
 // of 9 outweighs.  One thread per (i, j) of the box sets *bad when a pair of
-// zones of the box breaks the order.
+// zones of the box breaks the order: the entry point's contract, and more than
+// the sweep needs, which is that an earlier neighbour of the same plane
+// (dj <= 0) has di + 3 dj < 0 and so di + s dj < 0 for every s >= 3.
 __global__ void __launch_bounds__(256) k_ao_order(const P1 P, const Box b, unsigned int* bad) {
   const int64_t t = tid();
   if (t >= (int64_t)b.ni * b.nj) return;

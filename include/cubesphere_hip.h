@@ -148,6 +148,11 @@ int cs_init_problem(const cs_config* cfg, int32_t problem, uint64_t seed,
 int cs_create(const cs_config* cfg, cs_handle** out);
 int cs_destroy(cs_handle* h);
 
+/* The state to and from host arrays, finished on return.  Pageable arrays of
+ * 64 MiB (up) or 24 MiB (down) and more in all are copied by up to eight host
+ * threads, started for the call, through 32 MiB of pinned memory; up to two
+ * such sets a process stay allocated until the last handle is destroyed.
+ * Pinned arrays are copied directly. */
 int cs_upload_state(cs_handle* h, const double* U, const double* ent,
                     const double* Bxf, const double* Byf, const double* Bzf);
 int cs_download_state(cs_handle* h, double* U, double* ent, double* Bxf,
@@ -384,8 +389,11 @@ int cs_p1s_zone_geometry(const cs_config* cfg, double* centroid, double* volume,
  * inactive tri-corner zones get smallnum.  V_min_local / V_max_local are HOST
  * arrays of 9 (may be NULL).  stream: a hipStream_t, NULL = default stream.
  * The call waits on the stream once mid-way (the positivity limiter's
- * loop-order dependence) and at the end when the min/max are requested; calls
- * on one device share its work memory and are serialised. */
+ * loop-order dependence; when zones have lost all their slopes, again after
+ * every four sweeps of its replay) and at the end when the min/max are
+ * requested.  Calls on one device share its work memory: one call at a time
+ * puts its work on its stream, and an event makes the next call's stream wait
+ * for it.  A stream that is being captured is refused with CS_E_HIP. */
 typedef struct cs_p1_patch {
   int32_t ntp, nr, nghost;
   int32_t itri[4];                 /* itri_patch_LD, _RD, _RU, _LU (1 = tri-corner) */
@@ -470,10 +478,11 @@ int cs_build_volume_p12(const cs_config* cfg, const cs_volume_p12* out);
  * hold ten modes and whose v_centroid comes from the 27-point rule, plus
  * the ten basis moments (DEVICE, zone x 10).  Work memory, stream and the
  * host min/max as cs_limit_all_slopes_p1 (the call waits on the stream
- * mid-way and at the end).  CS_E_INVALID, with the outputs undefined, when the
- * stencil table breaks that order as the call runs it (level
- * (i+1) + 3 (j+1) + 9 (k+1)), which entries within two zones in i and j never
- * do; the cubed-sphere table reaches two, at the corner strips. */
+ * mid-way and at the end).  CS_E_INVALID, with the outputs undefined, when a
+ * stencil entry before its zone in that order is not on a lower level
+ * (i+1) + 3 (j+1) + 9 (k+1), or one after it not on a higher one, which entries
+ * within two zones in i and j never do; the cubed-sphere table reaches two, at
+ * the corner strips. */
 typedef struct cs_p12_patch {
   cs_p1_patch p1;
   const double* moments; /* Coef_Basis_Moments (zone, 10) */
@@ -496,8 +505,10 @@ int cs_limit_all_slopes_p12_timed(const cs_p12_patch* p, void* stream, float* ke
  * (Efx, Efy, Efz are zeroed over the zone range, as the routine does), no B0.
  * Device arrays in the layouts of cs_p1_patch; face outputs (S_*, Fluct_*,
  * EntFlux_*) in the face-B layout (0-g:N+g)^3-shaped [, 8]; dU_dt (zone, 8).
- * The call waits on the stream once (the count of faces re-pointed at the
- * tri-corners). */
+ * No wait on the stream: a caller that reads the outputs or reuses an input on
+ * another stream orders itself, as after every call that does not wait.  Calls
+ * on one device share its work memory, ordered between their streams by an
+ * event; a stream that is being captured is refused with CS_E_HIP. */
 typedef struct cs_p1_flux {
   int32_t ntp, nr, nghost, pad;
   double gamma, rhofloor, prsfloor, smallnum;

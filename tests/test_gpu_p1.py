@@ -439,3 +439,43 @@ def test_p1_sync_shared_gpu_matches_oracle():
                 assert not bad, (s, bad)
             else:
                 np.testing.assert_array_equal(G, As[s][k], err_msg=f"patch {s} {k}")
+
+
+def test_p1_calls_on_two_streams_share_the_work_memory():
+    """Reconstruction and facial fluxes of two patches of different size, put
+    on two streams in turn with no wait of the host between them beyond the
+    calls' own: the device's work memory, shared by all calls (and grown by the
+    larger patch's), passes from stream to stream by an event.  Every output
+    equals bit for bit that of the calls made one by one."""
+    print("\ntwo streams", flush=True)
+    dev = torch.device("cuda:0")
+    patches = []
+    for N, NR, s, seed in ((20, 6, 1, 2), (32, 8, 4, 5)):
+        prob, A = orc.p1_problem(N, NR, 4, sector=s, seed=seed, noise=0.8)
+        _, F = orc.p1_flux_problem(N, NR, 4, sector=s, seed=seed, noise=0.8)
+        patches.append((N, NR, prob, {k: torch.from_numpy(A[k]).to(dev) for k in cs.P1_ARRAYS},
+                        {k: torch.from_numpy(F[k]).to(dev) for k in cs.P1F_IN + cs.P1F_OUT}))
+    clone = lambda d: {k: v.clone() for k, v in d.items()}
+
+    def run(streams, rounds):
+        out = []
+        for (N, NR, prob, T, F), st in zip(patches, streams):
+            out.append([(clone(T), clone(F)) for _ in range(rounds)])
+        torch.cuda.synchronize()
+        for r in range(rounds):
+            for q, (N, NR, prob, _, _) in enumerate(patches):
+                T, F = out[q][r]
+                cs.limit_all_slopes_p1(N, NR, 4, prob, T, stream=streams[q], minmax=False)
+                cs.make_facial_fluxes_p1(N, NR, 4, prob, F, stream=streams[q])
+                if streams[0] is None:
+                    torch.cuda.synchronize()
+        torch.cuda.synchronize()
+        return out
+
+    want = run([None, None], 1)
+    got = run([torch.cuda.Stream(), torch.cuda.Stream()], 6)
+    for w, g in zip(want, got):
+        for rep in g:
+            for a, b in zip(w[0], rep):
+                for k in a:
+                    assert torch.equal(a[k].view(torch.uint8), b[k].view(torch.uint8)), k
