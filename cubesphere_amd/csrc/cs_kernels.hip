@@ -2608,6 +2608,16 @@ extern "C" int cs_time_kernel(cs_handle* h, int32_t kernel, int32_t iters, float
   return CS_OK;
 }
 
+// Not in the header, for the checks of the P1 stage: its face kernels march
+// face_pts and flux levels per workgroup on this handle (0: by the shell's
+// size).  Before the handle's first graph step.
+extern "C" int cs_p1_set_march(cs_handle* h, int32_t face_pts, int32_t flux) {
+  CHECK_H(h);
+  if (!h->p1 || h->graph || face_pts < 0 || flux < 0) { set_error("cs_p1_set_march: not now"); return CS_E_INVALID; }
+  p1s::set_march(h->p1, face_pts, flux);
+  return CS_OK;
+}
+
 extern "C" int cs_autotune(cs_handle* h, int32_t iters, int32_t* block_sizes) {
   CHECK_H(h);
   STAGE_PATH_ONLY(h, "cs_autotune");

@@ -24,6 +24,10 @@ struct Buf {
 int create(const cs_config* cfg, Stage** out, size_t* bytes);
 void destroy(Stage* S);
 
+// Levels per workgroup of the face kernels' marches in place of the rule's
+// (0: the rule's), so that long marches can be run on small shells.
+void set_march(Stage* S, int face_pts, int flux);
+
 // Steps 1 to 11 of the stage on buffer `in` (the exchange has run):
 // primitives, tri-corner face B, flattener, WENO, positivity (with its
 // bounded device-side replay), face-point B, constrained least squares, face

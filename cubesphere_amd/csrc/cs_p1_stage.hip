@@ -1968,8 +1968,13 @@ struct Stage {
   std::vector<void*> mem;
   Box all, wr, own, fx, fy, fz, ffx, ffy, ffz, ex, ey, ez;
   Marks* marks = nullptr;
+  int march_pts = 0, march_flux = 0;  // levels per workgroup of k_face_pts and k_flux; 0: march_levels
 };
 
+void set_march(Stage* S, int face_pts, int flux) {
+  S->march_pts = face_pts;
+  S->march_flux = flux;
+}
 void set_marks(Stage* S, Marks* m) { S->marks = m; }
 void mark_begin(Stage* S, hipStream_t st) {
   Marks* m = S->marks;
@@ -2195,7 +2200,7 @@ int front(Stage* S, const Buf& in_, double* const* F, double* const* Sp, double*
   k_clear_ent<<<kListBlocks, 256, 0, st>>>(D, S->wr, in, err);
   mark_end(S, st, CS_P1K_REPLAY);
   const int64_t nfpi = (D.N + 7 + kFpTI - 2) / (kFpTI - 1), nfpj = (D.N + 7 + kFpTJ - 2) / (kFpTJ - 1);
-  const int fpl = D.NR + 8, fpm = march_levels(fpl, 6 * nfpi * nfpj, kFpLevels);
+  const int fpl = D.NR + 8, fpm = S->march_pts ? S->march_pts : march_levels(fpl, 6 * nfpi * nfpj, kFpLevels);
   const int fpch = (fpl + fpm - 1) / fpm, fpnl = (fpl + fpch - 1) / fpch;
   mark_begin(S, st);
   k_face_pts<<<dim3((unsigned)(nfpi * nfpj * fpch), 6), kFpTI * kFpTJ, 0, st>>>(D, in, fpch, fpnl);
@@ -2205,8 +2210,8 @@ int front(Stage* S, const Buf& in_, double* const* F, double* const* Sp, double*
   mark_end(S, st, CS_P1K_CLSQ);
   const int64_t nfi = (D.N + 3 + kFluxTI - 2) / (kFluxTI - 1), nfj = (D.N + 3 + kFluxTJ - 2) / (kFluxTJ - 1);
   const int64_t tables = 6 * (int64_t)D.nf * D.nf * 35 * (int64_t)sizeof(double);
-  const int fll = D.NR + 4,
-            flm = march_levels(fll, 6 * nfi * nfj, tables > kInfinityCache ? kFluxLevelsBig : kFluxLevels);
+  const int fll = D.NR + 4, most = tables > kInfinityCache ? kFluxLevelsBig : kFluxLevels,
+            flm = S->march_flux ? S->march_flux : march_levels(fll, 6 * nfi * nfj, most);
   const int flch = (fll + flm - 1) / flm, flnl = (fll + flch - 1) / flch;
   mark_begin(S, st);
   k_flux<<<dim3((unsigned)(nfi * nfj * flch), 6), kFluxTI * kFluxTJ, 0, st>>>(D, F[0], F[1], F[2], Sp[0], Sp[1],

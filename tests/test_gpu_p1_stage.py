@@ -193,6 +193,37 @@ def test_p1_stage_march_chunks():
     _compare(cfg, got, ref, 1e-9)
 
 
+@pytest.mark.parametrize("name", ["shell8x20_hlld_imex", "C2_surface16_hlld_rk3", "shell20x9"])
+def test_p1_stage_march_lengths(name):
+    """The face kernels' marches at the lengths that large shells take (up to
+    eight levels a workgroup in k_face_pts and four or sixteen in k_flux) with
+    ragged last chunks, on small ones: two steps equal bit for bit those of
+    one-level marches, which test_p1_stage_matches_oracle compares with the
+    oracle."""
+    if name == "shell20x9":  # several blocks of columns in both directions
+        cfg, prob = cs.make_config(20, 9, 4, cs.RECON_P1ADP, cs.RS_HLLD, cs.EMF_LLF, cs.FP64, 2, cs.RBC_PAD,
+                                   cs.RMESH_UNIFORM, 1.0, 1.5), 2
+    else:
+        cfg, prob, _ = _cfg(name)
+    st0 = _state(cfg, prob, 0.0)
+    want = None
+    for pts, flux in ((1, 1), (2, 2), (3, 3), (5, 4), (8, 7), (16, 16)):
+        h = cs.CubeSphere(cfg)
+        try:
+            assert cs.lib().cs_p1_set_march(h.h, pts, flux) == 0
+            h.upload(st0)
+            h.dt = 1e-3
+            h.advance(2)
+            got = h.download(), h.dt
+        finally:
+            h.close()
+        if want is None:
+            want = got
+        for a, b in zip(got[0].arrays(), want[0].arrays()):
+            assert np.array_equal(a, b), (pts, flux)
+        assert got[1] == want[1]
+
+
 def test_p1_stage_long_replay_list():
     """The positivity replay with more zones on its list than its 512
     workgroups take in groups of 64 (a lane then redoes all fields of its
