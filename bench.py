@@ -770,8 +770,9 @@ def cpu_baseline_p1(max_seconds):
 # Algorithmic HBM bytes per work item of the P1 stage's launch groups (the
 # words an item must read or write once, data shared by neighbouring items
 # counted once): the work items are zones of the stated range, faces or edges.
-#   prim          zone (ghosts incl.): U + entropy read and written (18), V means
-#                 (9) and the magnetosonic speed (1) written
+#   prim          zone (ghosts incl.): U + entropy read (9); energy and entropy,
+#                 V means (9) and the magnetosonic speed written (12; the
+#                 conserved words that the conversion leaves are not)
 #   flatten       zone: speed, velocity, centroid, scale, pressure, three flag
 #                 passes (14 words)
 #   weno          zone of the WENO range: V means 9, centroid 3, scale 1,
@@ -798,7 +799,7 @@ def cpu_baseline_p1(max_seconds):
 #   imex          zone (ghosts incl.): U + entropy read and written, centroid
 #                 3, face B copied (3 + 3)
 #   cfl           owned zone: U + entropy 9 and scale 1 read, U 8 written
-P1K_BYTES = {"prim": 8 * 28, "flatten": 8 * 14, "weno": 8 * 41, "positivity": 8 * 41, "face_points": 8 * 18,
+P1K_BYTES = {"prim": 8 * 21, "flatten": 8 * 14, "weno": 8 * 41, "positivity": 8 * 41, "face_points": 8 * 18,
              "clsq": 8 * 45, "flux": 8 * 51, "edge": 8 * 15, "update_faces": 8 * 4, "update_zones": 8 * 61,
              "imex": 8 * 27, "cfl": 8 * 18}
 

@@ -2996,8 +2996,8 @@ __device__ __forceinline__ void wave_sync() {
 // (the Gram by FP64 MFMA) spent two broadcast instructions on each multiply-add
 // and eliminated both triangles: 64^2 x 25 1.34 -> 0.60 ms, 192^2 x 64 22.5 ->
 // 10.5 ms with k_e12, 49,644 operations a zone at 13.0 TFLOP/s.  What bounds
-// it now is FP64 issue at two waves per SIMD (1,500 multiply-adds and as many
-// broadcast moves per four zones); the point loop unrolled five-fold spills
+// it now is FP64 issue at two waves per SIMD (per lane 1,380 multiply-adds of
+// the Gram and 1,250 of the elimination, and 1,400 broadcast moves); the point loop unrolled five-fold spills
 // (0.69 ms at 64^2 x 25).  Against the system in 80-bit arithmetic its largest
 // relative error is 4.0e-15, the earlier form's 4.2e-15.
 constexpr int kSqStride = 484;    // LDS words per zone: 30 points of 16, and 4 against bank conflicts
