@@ -8,10 +8,10 @@
 // up to kWorkers threads move the words between the slots and the caller's
 // arrays, so the page faults are taken side by side.  The threads make no
 // runtime call (a thread's first one costs about 0.2 ms).
-// Milliseconds down (into a new array) / up, runtime's copy -> staged: 19 MB
-// 1.4 -> 1.1 / 0.6, 41 MB 3.0 -> 2.0 / 1.4, 109 MB 9.5 -> 3.6 / 3.8 -> 3.1,
-// 232 MB 22.8 -> 6.4 / 7.8 -> 6.2, 864 MB 81 -> 21.8 / 28.6 -> 22.2 (40 GB/s,
-// the link).  Below the thresholds the threads cost what they gain.
+// Milliseconds down (into a new array) / up, runtime's copy -> staged: 28 MiB
+// 2.4 -> 1.8, 48 MiB 4.2 -> 2.6, 125 MiB 12.1 -> 4.4 / 5.0 -> 3.7, 225 MiB
+// 22 -> 7.8 / 8.8 -> 6.3, 823 MiB 85 -> 23 / 32 -> 22 (40 GB/s, the link).
+// Below the thresholds the threads cost what they gain.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -29,10 +29,11 @@ namespace cs {
 
 constexpr int kWorkers = 8;                        // host threads of one transfer at most
 constexpr int kSlots = 16;                         // pinned slots
-constexpr size_t kSlotMin = (size_t)1 << 20;       // a slot: a 16th of the state, between
+constexpr size_t kSlotMin = (size_t)1 << 20;       // a slot: a 32nd of the state, between
 constexpr size_t kSlotMax = (size_t)2 << 20;       // 1 and 2 MiB
 constexpr size_t kStagedDown = (size_t)24 << 20;   // smallest staged transfers (transfer())
 constexpr size_t kStagedUp = (size_t)64 << 20;
+constexpr size_t kStagedAtOnce = (size_t)64 << 20; // smaller ones: from the second transfer on (StagingPool)
 
 struct Segment {
   char* dev;
@@ -40,18 +41,24 @@ struct Segment {
   size_t bytes;
 };
 
-// Pinned slots of one transfer at a time (32 MiB) with their events.
+inline size_t slot_bytes(size_t total) {
+  return std::min(kSlotMax, std::max(kSlotMin, total / 32 & ~(size_t)4095));
+}
+
+// Pinned slots of one transfer at a time (16 to 32 MiB) with their events.
 struct Staging {
   char* pin = nullptr;
+  size_t slot = 0;
   int device = -1;
   hipEvent_t ev[kSlots] = {};
   // for streams of device dev, whichever is the calling thread's: an event can
   // only be recorded on a stream of the device that was current when it was made
-  bool make(int dev) {
+  bool make(int dev, size_t bytes) {
     device = dev;
+    slot = bytes;
     int was = dev;
     bool ok = hipGetDevice(&was) == hipSuccess && (was == dev || hipSetDevice(dev) == hipSuccess);
-    ok = ok && hipHostMalloc((void**)&pin, kSlots * kSlotMax, hipHostMallocDefault) == hipSuccess;
+    ok = ok && hipHostMalloc((void**)&pin, kSlots * slot, hipHostMallocDefault) == hipSuccess;
     if (!ok) pin = nullptr;
     for (hipEvent_t& e : ev)
       if (ok && hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) {
@@ -70,8 +77,14 @@ struct Staging {
 };
 
 // The slot sets not in use, kept for the next transfer of any handle of their
-// device (allocating a set takes 2 ms): at most kIdleSets of them, released
-// when the last handle is destroyed.  A transfer owns its set alone.
+// device: at most kIdleSets of them, released when the last handle is
+// destroyed.  A transfer owns its set alone.  A MiB of slots costs 70 us to
+// have and give back, so a set has what its transfer needs, one that needs
+// more replaces it, and below 64 MiB, where a transfer gains less than its
+// set costs, the first one takes plain copies: a program that brings one
+// state back pays nothing (handle made, 28 MiB up, down, handle gone: 10.4 ms,
+// with a set of 32 MiB made at once 12.9), and one that goes on has its slots
+// from the second transfer.
 class StagingPool {
  public:
   static constexpr size_t kIdleSets = 2;
@@ -82,22 +95,28 @@ class StagingPool {
   void leave() {
     std::unique_ptr<Staging> drop[kIdleSets];
     std::lock_guard<std::mutex> l(mu_);
-    if (--handles_ == 0)
+    if (--handles_ == 0) {
       for (size_t q = 0; q < kIdleSets; ++q) drop[q] = std::move(idle_[q]);
+      small_ = 0;
+    }
   }
-  std::unique_ptr<Staging> take(hipStream_t st) {
+  std::unique_ptr<Staging> take(hipStream_t st, size_t total) {
+    const size_t slot = slot_bytes(total);
     int dev = 0;
     if (hipStreamGetDevice(st, &dev) != hipSuccess) {
       (void)hipGetLastError();
       return nullptr;
     }
+    std::unique_ptr<Staging> s;
     {
       std::lock_guard<std::mutex> l(mu_);
-      for (auto& s : idle_)
-        if (s && s->device == dev) return std::move(s);
+      for (auto& q : idle_)
+        if (q && q->device == dev && (!s || s->slot < q->slot)) std::swap(s, q);
+      if (s && s->slot >= slot) return s;
+      if (!s && total < kStagedAtOnce && small_++ == 0) return nullptr;
     }
-    std::unique_ptr<Staging> s(new (std::nothrow) Staging());
-    if (s && !s->make(dev)) s.reset();
+    s.reset(new (std::nothrow) Staging());
+    if (s && !s->make(dev, slot)) s.reset();
     return s;
   }
   void give(std::unique_ptr<Staging> s) {
@@ -112,6 +131,7 @@ class StagingPool {
  private:
   std::mutex mu_;
   int handles_ = 0;
+  unsigned small_ = 0;  // transfers below kStagedAtOnce that found no set
   std::unique_ptr<Staging> idle_[kIdleSets];
 };
 // never destroyed: the runtime may be gone by the time static objects are
@@ -134,9 +154,8 @@ struct Transfer {
   std::atomic<int64_t> moved[kSlots];  // the last chunk whose words a worker moved through the slot, plus one
   std::atomic<bool> stop{false};
 
-  Transfer(const Segment* s, int ns, size_t total, const Staging& S, bool to_host)
-      : seg(s), nseg(ns), slot(std::min(kSlotMax, std::max(kSlotMin, total / 16 & ~(size_t)4095))), pin(S.pin),
-        down(to_host) {
+  Transfer(const Segment* s, int ns, size_t slot_, const Staging& S, bool to_host)
+      : seg(s), nseg(ns), slot(slot_), pin(S.pin), down(to_host) {
     for (int q = 0; q < ns; ++q) n += (int64_t)((s[q].bytes + slot - 1) / slot);
     for (auto& m : moved) m.store(0, std::memory_order_relaxed);
     if (!down) opened.store(kSlots, std::memory_order_relaxed);
@@ -231,9 +250,9 @@ inline hipError_t transfer(hipStream_t st, const Segment* all, int nall, bool to
     }
   }
   std::unique_ptr<Staging> S;
-  if (total >= (to_host ? kStagedDown : kStagedUp)) S = staging_pool().take(st);
+  if (total >= (to_host ? kStagedDown : kStagedUp)) S = staging_pool().take(st, total);
   if (S) {
-    Transfer T(seg, nseg, total, *S, to_host);
+    Transfer T(seg, nseg, slot_bytes(total), *S, to_host);
     std::thread th[kWorkers];
     const int want = (int)std::min<int64_t>(std::min<int64_t>(kWorkers, T.n),
                                             std::max(1u, std::thread::hardware_concurrency()));

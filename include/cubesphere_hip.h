@@ -150,8 +150,9 @@ int cs_destroy(cs_handle* h);
 
 /* The state to and from host arrays, finished on return.  Pageable arrays of
  * 64 MiB (up) or 24 MiB (down) and more in all are copied by up to eight host
- * threads, started for the call, through 32 MiB of pinned memory; up to two
- * such sets a process stay allocated until the last handle is destroyed.
+ * threads, started for the call, through 16 to 32 MiB of pinned memory (below
+ * 64 MiB from the second such transfer on); up to two such sets a process stay
+ * allocated until the last handle is destroyed.
  * Pinned arrays are copied directly. */
 int cs_upload_state(cs_handle* h, const double* U, const double* ent,
                     const double* Bxf, const double* Byf, const double* Bzf);

@@ -24,7 +24,7 @@ def check(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("what", ["other_device", "fall_back", "pinned_arrays", "no_thread_memory"])
+@pytest.mark.parametrize("what", ["first_small", "other_device", "fall_back", "pinned_arrays", "no_thread_memory"])
 def test_transfer(check, what):
     r = subprocess.run([check, what], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0 and r.stdout.strip() == "ok", (r.returncode, r.stdout, r.stderr[-300:])

@@ -48,9 +48,46 @@ struct State {
   bool same() const { return dev[0] == host[0] && dev[1] == host[1] && dev[2] == host[2]; }
 };
 
+// past the first small transfer, which has no slots yet, with slots for any size
+static bool warm(FakeStream* st) {
+  State S(130);
+  return transfer(st, S.seg, 3, true) == hipSuccess;
+}
+
+// slots from the second transfer on below 64 MiB, at once from there, anew after the last handle
+static int first_small() {
+  FakeStream st{0};
+  State S(25), L(64);
+  for (int round = 0; round < 2; ++round) {
+    for (int n = 0; n < 3; ++n) {
+      S.fill(true, n);
+      fake().direct = fake().staged = 0;
+      if (transfer(&st, S.seg, 3, true) != hipSuccess || !S.same()) return fail("words lost");
+      if ((n == 0 ? fake().direct : fake().staged) != S.bytes()) return fail("slots not from the second transfer");
+    }
+    const size_t few = fake().pin.begin()->second;
+    if (few > 16 * (size_t)(1 << 20)) return fail("more slots than the transfer needs");
+    L.fill(true, 9);
+    fake().direct = fake().staged = 0;
+    if (transfer(&st, L.seg, 3, true) != hipSuccess || !L.same()) return fail("words lost");
+    if (fake().staged != L.bytes()) return fail("a large transfer not staged");
+    if (fake().pin.size() != 1 || fake().pin.begin()->second <= few) return fail("the small set was not replaced");
+    staging_pool().leave();
+    if (!fake().pin.empty()) return fail("slots kept after the last handle");
+    staging_pool().enter();
+    fake().direct = fake().staged = 0;
+    if (transfer(&st, L.seg, 3, true) != hipSuccess || fake().staged != L.bytes())
+      return fail("the first large transfer not staged");
+    staging_pool().leave();
+    staging_pool().enter();
+  }
+  return 0;
+}
+
 // the handle's stream on a device that is not the calling thread's
 static int other_device() {
   FakeStream st{1};
+  if (!warm(&st)) return fail("a transfer of a handle on another device failed");
   for (bool down : {true, false}) {
     State S(down ? 25 : 66);
     S.fill(down, 3);
@@ -66,6 +103,7 @@ static int other_device() {
 // staging that fails half way: the plain copies take over, and no error is left behind
 static int fall_back() {
   FakeStream st{0};
+  if (!warm(&st)) return fail("failed");
   for (bool down : {true, false}) {
     State S(down ? 40 : 80);
     S.fill(down, 5);
@@ -80,6 +118,7 @@ static int fall_back() {
 // arrays that the runtime can reach by itself: its own copies, no pass through the slots
 static int pinned_arrays() {
   FakeStream st{0};
+  if (!warm(&st)) return fail("failed");
   for (bool down : {true, false})
     for (int pin = 0; pin < 3; ++pin) {  // none, one, all of them
       State S(down ? 25 : 66);
@@ -118,8 +157,7 @@ static int pinned_arrays() {
 // no memory for any thread's start, or after the first or the third (the slots are in the pool)
 static int no_thread_memory() {
   FakeStream st{0};
-  State warm(25);
-  if (transfer(&st, warm.seg, 3, true) != hipSuccess) return fail("failed");
+  if (!warm(&st)) return fail("failed");
   for (bool down : {true, false})
     for (int have : {0, 1, 3}) {
       State S(down ? 25 : 66);
@@ -138,6 +176,7 @@ int main(int argc, char** argv) {
   int rc = 2;
   staging_pool().enter();
   if (what == "other_device") rc = other_device();
+  if (what == "first_small") rc = first_small();
   if (what == "fall_back") rc = fall_back();
   if (what == "pinned_arrays") rc = pinned_arrays();
   if (what == "no_thread_memory") rc = no_thread_memory();
