@@ -479,3 +479,32 @@ def test_p1_calls_on_two_streams_share_the_work_memory():
             for a, b in zip(w[0], rep):
                 for k in a:
                     assert torch.equal(a[k].view(torch.uint8), b[k].view(torch.uint8)), k
+
+
+def test_p1_calls_refuse_a_captured_stream():
+    """The calls that share work memory return an error on a stream that is
+    being captured, before anything is put on it: the capture goes on, and the
+    calls work on the stream afterwards."""
+    N, NR = 8, 3
+    print("\ncaptured stream", flush=True)
+    dev = torch.device("cuda:0")
+    prob, A = orc.p1_problem(N, NR, 4, sector=0, seed=1)
+    _, F0 = orc.p1_flux_problem(N, NR, 4, sector=0, seed=1)
+    T = {k: torch.from_numpy(A[k]).to(dev) for k in cs.P1_ARRAYS}
+    F = {k: torch.from_numpy(F0[k]).to(dev) for k in cs.P1F_IN + cs.P1F_OUT}
+    x = torch.zeros(4, device=dev)
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        st = torch.cuda.current_stream()
+        x += 1.0
+        with pytest.raises(cs.CsError, match="captured"):
+            cs.make_facial_fluxes_p1(N, NR, 4, prob, F, stream=st)
+        with pytest.raises(cs.CsError, match="captured"):
+            cs.limit_all_slopes_p1(N, NR, 4, prob, T, stream=st)
+    for _ in range(3):
+        g.replay()
+    cs.make_facial_fluxes_p1(N, NR, 4, prob, F, stream=st)
+    cs.limit_all_slopes_p1(N, NR, 4, prob, T, stream=st)
+    torch.cuda.synchronize()
+    assert torch.equal(x, torch.full_like(x, 3.0))
